@@ -329,11 +329,12 @@ __device__ __forceinline__ void fused_first_tile(const fnkv_datc_attend_args & a
     __builtin_amdgcn_sched_barrier(0);
     float sn, cs;
     rope_angle(sn, cs, pq, pa.theta_scale, lane);
+    const rope_pairs rp = rope_pairs_of(sn, cs, lane);
 #pragma unroll
     for (int32_t i = 0; i < kPer; ++i) {
         const int32_t h = kPer * wave + i;
         float y[4];
-        norm_rope_apply(y, xq[i], gq, sn, cs, lane);
+        norm_rope_apply(y, xq[i], gq, rp, lane);
         const uint2 q4 = pack4_f16(y, 1.0f / 16.0f);
         reinterpret_cast<uint2 *>(ql + h * kD)[lane] = q4;
         if (b == 0) {

@@ -5,6 +5,7 @@
 // (ggml-impl.h:414-438). Lane l holds values 4 l .. 4 l + 3; the 8 lanes of a block reduce amax with cross-lane max.
 #pragma once
 
+#include "lanes.h"
 #include "layout.h"
 
 #include <hip/hip_fp16.h>
@@ -61,17 +62,13 @@ __device__ __forceinline__ void quantize_q8_0(const float (&x)[4], uint32_t & pa
     for (int32_t e = 0; e < 4; ++e) {
         last_nan = x[e] != x[e] ? base + e : last_nan;
     }
-    last_nan = max(last_nan, __shfl_xor(last_nan, 1));
-    last_nan = max(last_nan, __shfl_xor(last_nan, 2));
-    last_nan = max(last_nan, __shfl_xor(last_nan, 4));
+    last_nan = max8(last_nan);
     float amax = 0.0f;
 #pragma unroll
     for (int32_t e = 0; e < 4; ++e) {
         amax = base + e > last_nan ? fmaxf(amax, __builtin_fabsf(x[e])) : amax;
     }
-    amax = fmaxf(amax, __shfl_xor(amax, 1));
-    amax = fmaxf(amax, __shfl_xor(amax, 2));
-    amax = fmaxf(amax, __shfl_xor(amax, 4));
+    amax = max8(amax);
     if (last_nan == kQK - 1) {
         amax = __builtin_nanf("");
     }
@@ -99,10 +96,7 @@ __device__ __forceinline__ void quantize_kv8(const float (&x)[4], uint32_t & pac
 #pragma clang fp contract(off)
     float amax = fmaxf(fmaxf(__builtin_fabsf(x[0]), __builtin_fabsf(x[1])),
                        fmaxf(__builtin_fabsf(x[2]), __builtin_fabsf(x[3])));
-    amax = fmaxf(amax, __shfl_xor(amax, 1));
-    amax = fmaxf(amax, __shfl_xor(amax, 2));
-    amax = fmaxf(amax, __shfl_xor(amax, 4));
-    amax = fmaxf(amax, __shfl_xor(amax, 8));
+    amax = max16(amax);
     const __half h = __float2half_rn(__fdiv_rn(amax, 127.0f));
     const float sv = __half2float(h);
     packed = 0;

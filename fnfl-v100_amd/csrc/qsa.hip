@@ -10,8 +10,8 @@
 //   2. the sparse decode launch (each row its own splits);
 //   3. the merge with the gated epilogue.
 // At most 16 query heads a KV head skip step 1: the sparse launch forms each row's query heads in LDS while the row's
-// selection builds, and every workgroup that reads a new cell's tile writes that cell first (a row's own cell also
-// by its owner when no workgroup reads it; fused_prep, decode.hip). Workgroups that write the same cell store the same
+// page-table words arrive, and every workgroup that reads a new cell's block writes that cell first (a row's own cell
+// also by its owner when no workgroup reads it; fused_prep, gather.h). Workgroups that write the same cell store the same
 // bytes, and the arithmetic is the prepare kernel's, so the outputs are bitwise those of the three launches.
 // Differences from the reference's kernel: the query enters the matrix cores as two fp16 parts (the reference keeps q
 // in F32; hi + lo carries it to about 2^-22 relative, and the output meets the reference checker's 1e-5 normalized
@@ -19,6 +19,7 @@
 #include "../../include/fnkv.h"
 #include "common.h"
 #include "decode_common.h"
+#include "gather.h"
 #include "rope.h"
 
 #include <hip/hip_runtime.h>
@@ -136,7 +137,12 @@ int qsa_launch(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_t T, i
     uint16_t * q16 = reinterpret_cast<uint16_t *>(w + sp);
     uint16_t * q16_lo = q16 + int64_t(T) * hq * 256;
     // every check of the sparse launch is made here too, before the prepare is enqueued: a refusal enqueues nothing
-    sparse_gate gate = {qfull + 256, 512, out, codes, scales};
+    out_args gate;
+    gate.gate = qfull + 256;
+    gate.gate_stride = 512;
+    gate.out_f32 = out;
+    gate.codes = codes;
+    gate.act_scales = scales;
     if (T <= 0 || T > kSelMaxRows || depth < 0 || layer < 0 || layer >= p->layers() || slot < 0 ||
         slot >= p->pages().n_slots() || depth + T > p->mapped_cells(slot) || depth + T > kSelMaxCells ||
         G > FNKV_MAX_ROWS || body == nullptr || offsets == nullptr || (reinterpret_cast<uintptr_t>(body) & 3) != 0 ||

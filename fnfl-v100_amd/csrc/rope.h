@@ -3,6 +3,7 @@
 // run of 32 values.
 #pragma once
 
+#include "lanes.h"
 #include "mfma.h"
 
 #include <hip/hip_runtime.h>
@@ -19,7 +20,7 @@ constexpr float kRmsEps = 1e-6f; // fn/model/shapes.h:35 rms_eps
 // 4 lane .. 4 lane + 3. Rotation pair i (< 32) is dims i and i + 32; its angle is its plane's position times
 // theta_scale^i as the F32 product chain, the plane picked by the sector rule (sections 11, 11, 10, 0).
 // Split in three for callers that issue the loads early: rope_pos (the lane's plane position), rope_angle (the lane's
-// pair angle as sin / cos, shared by every row at one position), norm_rope_apply (the norm and rotation of a loaded row).
+// pair angle as sin / cos, shared by every row at one position; rope_pairs_of spreads it), norm_rope_apply (the norm and rotation of a loaded row).
 __device__ __forceinline__ int32_t rope_plane(int32_t lane) {
     const int32_t sector = lane & 31;
     return sector % 3 == 1 && sector < 33   ? 1
@@ -48,17 +49,30 @@ __device__ __forceinline__ void rope_angle(float & s, float & c, int32_t p, floa
     sincosf(theta, &s, &c);
 }
 
-__device__ __forceinline__ void norm_rope_apply(float (&y)[4], const float4 x, const float4 g, float s, float c,
+// the cosines and sines of this lane's four pairs (lanes 0..15: dims 4 lane .. + 3 and their partners), from the lanes
+// that formed them: one set serves every row at the position
+struct rope_pairs {
+    float c[4], s[4];
+};
+__device__ __forceinline__ rope_pairs rope_pairs_of(float s, float c, int32_t lane) {
+    rope_pairs p;
+#pragma unroll
+    for (int32_t e = 0; e < 4; ++e) {
+        const int32_t pair = 4 * (lane & 7) + e;
+        p.c[e] = __shfl(c, pair, 64);
+        p.s[e] = __shfl(s, pair, 64);
+    }
+    return p;
+}
+
+__device__ __forceinline__ void norm_rope_apply(float (&y)[4], const float4 x, const float4 g, const rope_pairs & p,
                                                 int32_t lane) {
 #pragma clang fp contract(off)
     float ss = x.x * x.x;
     ss = __builtin_fmaf(x.y, x.y, ss);
     ss = __builtin_fmaf(x.z, x.z, ss);
     ss = __builtin_fmaf(x.w, x.w, ss);
-#pragma unroll
-    for (int32_t o = 32; o > 0; o >>= 1) {
-        ss += __shfl_xor(ss, o, 64);
-    }
+    ss = wave_sum(ss);
     const float r = 1.0f / sqrtf(ss * (1.0f / 256.0f) + kRmsEps);
     y[0] = x.x * r * g.x;
     y[1] = x.y * r * g.y;
@@ -67,15 +81,10 @@ __device__ __forceinline__ void norm_rope_apply(float (&y)[4], const float4 x, c
     // dims 0..31 sit in lanes 0..7, their partners 32..63 in lanes 8..15
 #pragma unroll
     for (int32_t e = 0; e < 4; ++e) {
-        const int32_t pair = 4 * (lane & 7) + e;
-        const float ce = __shfl(c, pair, 64);
-        const float se = __shfl(s, pair, 64);
-        const float other = __shfl_xor(y[e], 8, 64);
-        if (lane < 8) {
-            y[e] = y[e] * ce - other * se;
-        } else if (lane < 16) {
-            y[e] = other * se + y[e] * ce;
-        }
+        const float other = dpp_f<kDppRor + 8>(y[e]); // lane ^ 8
+        const float lo = y[e] * p.c[e] - other * p.s[e];
+        const float hi = other * p.s[e] + y[e] * p.c[e];
+        y[e] = lane < 8 ? lo : lane < 16 ? hi : y[e];
     }
 }
 
@@ -85,7 +94,7 @@ __device__ __forceinline__ void norm_rope(float (&y)[4], const float * src, cons
     const float4 g = reinterpret_cast<const float4 *>(w)[lane];
     float s, c;
     rope_angle(s, c, rope_pos(pos, stride, col, lane), ts, lane);
-    norm_rope_apply(y, x, g, s, c, lane);
+    norm_rope_apply(y, x, g, rope_pairs_of(s, c, lane), lane);
 }
 
 __device__ __forceinline__ uint2 pack4_f16(const float (&x)[4], float scale) {
@@ -106,9 +115,13 @@ __device__ __forceinline__ void act_run(const float (&y)[N], int8_t (&q)[N], flo
     for (int32_t e = 0; e < N; ++e) {
         amax = fmaxf(amax, fabsf(y[e]));
     }
+    if constexpr (WIDTH == 8) {
+        amax = max8(amax);
+    } else {
 #pragma unroll
-    for (int32_t o = WIDTH / 2; o > 0; o >>= 1) {
-        amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+        for (int32_t o = WIDTH / 2; o > 0; o >>= 1) {
+            amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+        }
     }
     const float d = amax / 127.0f;
     const float id = amax > 0.0f ? 127.0f / amax : 0.0f;
@@ -120,9 +133,13 @@ __device__ __forceinline__ void act_run(const float (&y)[N], int8_t (&q)[N], flo
         q[e] = static_cast<int8_t>(c);
         sum += c;
     }
+    if constexpr (WIDTH == 8) {
+        sum = sum8(sum);
+    } else {
 #pragma unroll
-    for (int32_t o = WIDTH / 2; o > 0; o >>= 1) {
-        sum += __shfl_xor(sum, o, 64);
+        for (int32_t o = WIDTH / 2; o > 0; o >>= 1) {
+            sum += __shfl_xor(sum, o, 64);
+        }
     }
     ds[0] = d;
     ds[1] = d * static_cast<float>(sum);

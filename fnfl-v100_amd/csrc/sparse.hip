@@ -4,23 +4,17 @@
 // production decode path (attn::attend over the body, fn/kernels/qsa/attend.h:97-141, cell expansion
 // attend.cu:405-421), here over the Q8_0 / KV8 pool.
 //
-// How (MI355X):
-//   * The decode kernels (decode_kernel<1, true>, decode_rows_kernel<NT, true>) walk the selection's tiles instead of
-//     a range of consecutive cells. Each workgroup rebuilds the selection in LDS from the bodies (sparse_build: row
-//     t's 8 bits a 32-cell tile, one a 4-cell block; the tiles any row selected in ascending order, by a block-wide
-//     scan) and takes entries s * S .. s * S + S - 1 of that list; a lane's four scores of a tile half are one 4-cell
-//     block, so the row's mask enters the softmax as one bit a half, the causal limit (own position) as in the dense
-//     launch. The rows' own cells are written by the workgroup that reads their tile (split 0 when no row selects
-//     it). A split past the list's end returns at once; split 0 of head 0 stores the list's length.
-//   * merge_kernel folds the splits that ran (it reads the list's length).
-// Tiles are read whole (17,408 B) even when one block of them is selected: the pool's layout is tile-granular, and
-// selections that cluster (sinks, local windows, topical runs) share tiles across blocks and rows.
+// The kernel is gather.hip's (eight selected blocks a virtual tile, each lane loading its own block's bytes); here are
+// the launches' checks and plans. A row's new cell is written by the workgroups that read its block (several rows
+// without a prepare: by an append launch first, since a row may read an earlier row's cell); the rows of one launch run
+// side by side, each as its own splits, and merge_kernel folds the splits that held some of a row's tiles.
 #include "../../include/fnkv.h"
 #include "common.h"
 #include "layout.h"
 #include "mfma.h"
 #include "q8_0.h"
 #include "decode_common.h"
+#include "gather.h"
 
 #include <hip/hip_runtime.h>
 
@@ -31,40 +25,72 @@
 
 namespace fnkv {
 
-#ifdef FNKV_TIMING
-uint64_t * timing_buffer();
-#endif
-
-// The launch shape of a sparse step: each of the T rows runs as its own n_splits splits (a row's list: at most its
-// 513 tiles), the entries a split takes, the partials of every row.
+// The launch shape of `rows` rows, the deepest at position last: each row's splits, whether a wave takes several tiles,
+// and the partials of every split (a row of one split writes none, its region is unused).
+//   * Decode rows (at most kSelMaxRows): one virtual tile a wave, the row's at most 65 tiles over at most 17 splits. A
+//     step has few rows, so its time is one tile's latency, and fewer, longer splits leave the device idle.
+//   * Prompt rows: the splits that bring the launch to two workgroups a CU (what its LDS lets run at once), one from
+//     512 (row, head tile) pairs on: such rows need no partials and no merge.
 struct sparse_plan {
-    int32_t n_max = 0, per_split = 0, n_splits = 0;
-    int64_t po_off = 0, pml_off = 0, bytes = 0;
+    int32_t n_splits = 0;
+    bool many = false;
+    int64_t pml_off = 0, bytes = 0;
 };
-sparse_plan plan_sparse(const kv_pool & p, int64_t depth, int32_t T, int32_t G) {
+sparse_plan plan_sparse(const kv_pool & p, int64_t last, int32_t rows, int32_t G) {
     sparse_plan pl;
-    const int32_t n_tiles = static_cast<int32_t>((depth + T + kTileTokens - 1) / kTileTokens);
-    pl.n_max = std::min(n_tiles, kSelTopBlocks + 1); // a row's blocks' tiles and its tail's
-    int32_t want = std::max(1, device_cus(p.device()) / (p.h_kv() * T));
-    static const int32_t want_knob = env_int_once("FNKV_SPARSE_WANT", 0); // splits a row and head, for measurement
-    if (want_knob > 0) {
-        want = want_knob;
+    // the deepest row's blocks and one tail entry (which rows have a tail follows from each row's own position)
+    const int32_t entries = sel_shape(static_cast<int32_t>(std::min<int64_t>(last, kSelMaxCells))).K + 1;
+    const int32_t full = (entries + 8 * kGatherWaves - 1) / (8 * kGatherWaves);
+    pl.n_splits = full;
+    if (rows > kSelMaxRows) {
+        const int64_t pairs = int64_t(rows) * p.h_kv() * ((G + 15) / 16);
+        pl.n_splits = static_cast<int32_t>(
+            std::min<int64_t>(full, std::max<int64_t>(1, 2 * int64_t(device_cus(p.device())) / pairs)));
     }
-    pl.per_split = std::min(64, std::max(1, (pl.n_max + want - 1) / want));
-    pl.n_splits = (pl.n_max + pl.per_split - 1) / pl.per_split;
+    pl.many = pl.n_splits < full;
     auto up16 = [](int64_t x) { return (x + 15) & ~int64_t(15); };
-    pl.po_off = up16(int64_t(T) * 4); // each row's list length first
-    pl.pml_off = up16(pl.po_off + int64_t(T) * pl.n_splits * p.h_kv() * G * kHeadDim * 4);
-    pl.bytes = up16(pl.pml_off + int64_t(T) * pl.n_splits * p.h_kv() * G * 2 * 4);
+    const int64_t prows = int64_t(rows) * pl.n_splits * p.h_kv() * G;
+    pl.pml_off = prows * kHeadDim * 4;
+    pl.bytes = up16(pl.pml_off + prows * 2 * 4);
     return pl;
 }
 
-// The sparse launch (validation, the decode kernels' sparse instantiation, the merge); `gate` set: the merge writes
-// the gated F32 output and its activation format instead of the fp16 out. Returns a status; nothing is enqueued
-// unless it is FNKV_OK.
+// the kernel, then the merge when a row has several splits
+int sparse_enqueue(const kv_pool & p, int32_t slot, const sparse_plan & pl, gather_args & a, void * ws, hipStream_t st) {
+    a.pv = p.view();
+    a.table = a.pv.table + int64_t(slot) * a.pv.table_stride;
+    a.n_splits = pl.n_splits;
+    a.many = pl.many ? 1 : 0;
+    a.head_tiles = (a.G + 15) / 16;
+    a.po = static_cast<float *>(ws);
+    a.pml = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + pl.pml_off);
+    launch_gather(p.device(), a, st);
+    if (pl.n_splits > 1) {
+        merge_args m;
+        m.po = a.po;
+        m.pml = a.pml;
+        m.fin = a.fin;
+        m.T = 1; // the rows fold as sequences of one step token each
+        m.G = a.G;
+        m.hq = a.hq;
+        m.R = a.G;
+        m.h_kv = p.h_kv();
+        m.n_seq = a.T;
+        m.sel_splits = pl.n_splits;
+        m.depth = a.depth;
+        m.depth_dev = a.depth_dev;
+        m.cap[0] = a.cap;
+        m.T_dev = a.T;
+        launch_merge(m, st);
+    }
+    return hipGetLastError() == hipSuccess ? FNKV_OK : FNKV_ERR_HIP;
+}
+
+// The sparse launch of decode rows; `gate` set: the gated F32 output and its activation format instead of the fp16
+// out. Returns a status; nothing is enqueued unless it is FNKV_OK.
 int sparse_launch(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_t T, int32_t layer, int32_t hq, float scale,
                   const void * q, const void * body, const void * offsets, const void * k_new, const void * v_new,
-                  int32_t new_dtype, void * out, const sparse_gate * gate, void * ws, int64_t ws_bytes,
+                  int32_t new_dtype, void * out, const out_args * gate, void * ws, int64_t ws_bytes,
                   hipStream_t st, const char * who, const fused_prep * fp, const dev_depth * dd,
                   const uint16_t * q_lo) {
     const kv_pool * p = pool_of(pool);
@@ -99,13 +125,11 @@ int sparse_launch(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_t T
         set_error(name + ": q, out and ws must be 16-byte aligned, body and offsets 4-byte aligned");
         return FNKV_ERR_ARG;
     }
-    const sparse_plan pl = plan_sparse(*p, depth, T, G);
+    const sparse_plan pl = plan_sparse(*p, ctx - 1, T, G);
     if (ws_bytes < pl.bytes) {
         set_error(name + ": workspace too small");
         return FNKV_ERR_ARG;
     }
-    uint8_t * w = static_cast<uint8_t *>(ws);
-
     // several rows: their new cells first (a row may read an earlier row's new cell; the rows run side by side); one
     // row: the launch writes it, by the split that reads its tile
     if (fp != nullptr && (G > 16 || fp->rows != T)) {
@@ -119,156 +143,61 @@ int sparse_launch(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_t T
             return FNKV_ERR_HIP;
         }
     }
-    dec_args a;
-    a.pv = p->view();
-    a.q = static_cast<const uint16_t *>(q);
-    a.k_new = T == 1 ? k_new : nullptr;
-    a.v_new = T == 1 ? v_new : nullptr;
-    a.new_f32 = new_dtype == FNKV_F32 ? 1 : 0;
-    a.po = reinterpret_cast<float *>(w + pl.po_off);
-    a.pml = reinterpret_cast<float *>(w + pl.pml_off);
-    a.c2 = scale * 1.4426950408889634f;
+    gather_args a = {};
     a.layer = layer;
     a.T = T;
     a.G = G;
     a.hq = hq;
-    a.R = G * T; // each row's view takes G of them
-    a.n_seq = 1;
-    a.split_tokens = 0;
-    a.strided = 0;
-    for (int32_t i = 0; i < FNKV_MAX_SEQS; ++i) {
-        a.slot[i] = slot;
-        a.ctx[i] = ctx;
-    }
-    a.split0[0] = 0;
-    for (int32_t i = 1; i <= FNKV_MAX_SEQS; ++i) {
-        a.split0[i] = pl.n_splits;
-    }
-    a.sel_body = static_cast<const uint32_t *>(body);
-    a.sel_n = reinterpret_cast<int32_t *>(w);
-    a.sel_split = pl.per_split;
-    if (fp != nullptr) {
-        a.fp = *fp;
-    }
-    a.q_lo = q_lo;
+    a.depth = depth;
+    a.cap = ctx;
     if (dd != nullptr) {
         a.depth_dev = dd->depth;
         a.err = dd->err;
     }
-#ifdef FNKV_TIMING
-    a.ts = timing_buffer();
-#endif
-    launch_decode_sparse(*p, (G + 15) / 16,
-                         dim3(static_cast<uint32_t>(pl.n_splits), static_cast<uint32_t>(p->h_kv()),
-                              static_cast<uint32_t>(T)),
-                         a, st);
-    merge_args m;
-    m.po = a.po;
-    m.pml = a.pml;
-    m.out = static_cast<uint16_t *>(out);
-    // the rows fold as sequences of one step token each ([row][split] partials, row r's out at row r)
-    m.T = 1;
-    m.G = G;
-    m.hq = hq;
-    m.R = G;
-    m.h_kv = p->h_kv();
-    m.n_seq = T;
-    for (int32_t i = 0; i <= FNKV_MAX_SEQS; ++i) {
-        m.split0[i] = (i < T ? i : T) * pl.n_splits;
+    a.body = static_cast<const uint32_t *>(body);
+    a.q = static_cast<const uint16_t *>(q);
+    a.q_lo = q_lo;
+    if (fp != nullptr) {
+        a.fp = *fp;
+    } else if (T == 1) {
+        a.k_new = k_new;
+        a.v_new = v_new;
+        a.new_f32 = new_dtype == FNKV_F32 ? 1 : 0;
     }
-    m.sel_n = a.sel_n;
-    m.sel_split = pl.per_split;
-    if (dd != nullptr) {
-        m.depth_dev = dd->depth;
-        m.cap[0] = ctx;
-        m.T_dev = T;
-    }
+    a.c2 = scale * 1.4426950408889634f;
     if (gate != nullptr) {
-        m.gate = gate->gate;
-        m.gate_stride = gate->stride;
-        m.out_f32 = gate->out_f32;
-        m.codes = gate->codes;
-        m.act_scales = gate->scales;
+        a.fin = *gate;
+    } else {
+        a.fin.out = static_cast<uint16_t *>(out);
     }
-    launch_merge(m, st);
-    if (hipGetLastError() != hipSuccess) {
+    if (sparse_enqueue(*p, slot, pl, a, ws, st) != FNKV_OK) {
         set_error(name + ": launch failed");
         return FNKV_ERR_HIP;
     }
     return FNKV_OK;
 }
 
-// Prompt rows (qsp_attend): rows row0 .. row0 + n - 1 of a prompt half at positions pos0 + row, each over its own
-// selection body (the slab layout), q16 the rows' prepared fp16 queries [n][hq][256], then the gated merge into the
-// F32 (optional) and fp16 outputs. The caller has checked the arguments; ws holds prompt_ws_bytes(pool, cells, n, hq).
-int64_t prompt_ws_bytes(const kv_pool & p, int64_t cells, int32_t n, int32_t G) {
-    return plan_sparse(p, cells - n, n, G).bytes;
+// Prompt rows (qsp_attend): each over its own selection body (the slab layout), its query heads formed by the launch.
+// The caller has checked the arguments; ws holds prompt_ws_bytes.
+int64_t prompt_ws_bytes(const kv_pool & p, int64_t pos0, int32_t rows, int32_t G) {
+    return plan_sparse(p, pos0 + rows - 1, rows, G).bytes;
 }
 
-int prompt_launch(const kv_pool & p, int32_t slot, int32_t layer, int32_t pos0, int32_t row0, int32_t n, int32_t hq,
-                  const uint16_t * q16, const uint32_t * body, const int32_t * offsets, const float * gate,
-                  float * out_f32, uint16_t * out16, uint32_t * err, void * ws, hipStream_t st) {
-    const int32_t G = hq / p.h_kv();
-    const int64_t last = int64_t(pos0) + row0 + n; // cells the chunk's last row sees
-    const sparse_plan pl = plan_sparse(p, last - n, n, G);
-    uint8_t * w = static_cast<uint8_t *>(ws);
-    dec_args a;
-    a.pv = p.view();
-    a.q = q16;
-    a.k_new = nullptr;
-    a.v_new = nullptr;
-    a.new_f32 = 0;
-    a.po = reinterpret_cast<float *>(w + pl.po_off);
-    a.pml = reinterpret_cast<float *>(w + pl.pml_off);
-    a.c2 = (1.0f / 16.0f) * 1.4426950408889634f;
+int prompt_launch(const kv_pool & p, int32_t slot, int32_t layer, int32_t pos0, int32_t rows, int32_t hq,
+                  const uint32_t * body, const int32_t * offsets, const fused_prep & fp, const out_args & fin, void * ws,
+                  hipStream_t st) {
+    gather_args a = {};
     a.layer = layer;
-    a.T = n;
-    a.G = G;
+    a.T = rows;
+    a.G = hq / p.h_kv();
     a.hq = hq;
-    a.R = G * n;
-    a.n_seq = 1;
-    a.split_tokens = 0;
-    a.strided = 0;
-    for (int32_t i = 0; i < FNKV_MAX_SEQS; ++i) {
-        a.slot[i] = slot;
-        a.ctx[i] = last;
-    }
-    a.split0[0] = 0;
-    for (int32_t i = 1; i <= FNKV_MAX_SEQS; ++i) {
-        a.split0[i] = pl.n_splits;
-    }
-    a.sel_body = body;
-    a.sel_n = reinterpret_cast<int32_t *>(w);
-    a.sel_split = pl.per_split;
-    a.sel_offsets = offsets;
-    a.sel_row0 = row0;
-#ifdef FNKV_TIMING
-    a.ts = timing_buffer();
-#endif
-    launch_decode_sparse(p, (G + 15) / 16,
-                         dim3(static_cast<uint32_t>(pl.n_splits), static_cast<uint32_t>(p.h_kv()),
-                              static_cast<uint32_t>(n)),
-                         a, st);
-    merge_args m;
-    m.po = a.po;
-    m.pml = a.pml;
-    m.out = nullptr;
-    m.T = 1;
-    m.G = G;
-    m.hq = hq;
-    m.R = G;
-    m.h_kv = p.h_kv();
-    m.n_seq = n;
-    m.uniform_splits = pl.n_splits;
-    m.sel_n = a.sel_n;
-    m.sel_split = pl.per_split;
-    m.gate = gate;
-    m.gate_stride = 512;
-    m.out_f32 = out_f32;
-    m.out16 = out16;
-    m.err = err;
-    launch_merge(m, st);
-    return hipGetLastError() == hipSuccess ? FNKV_OK : FNKV_ERR_HIP;
+    a.depth = pos0;
+    a.body = body;
+    a.offsets = offsets;
+    a.fp = fp;
+    a.c2 = (1.0f / 16.0f) * 1.4426950408889634f;
+    a.fin = fin;
+    return sparse_enqueue(p, slot, plan_sparse(p, int64_t(pos0) + rows - 1, rows, a.G), a, ws, st);
 }
 
 } // namespace fnkv
@@ -282,7 +211,7 @@ int64_t fnkv_sparse_workspace_bytes(const fnkv_pool * pool, int64_t depth, int32
     if (p == nullptr || T <= 0 || T > fnkv::kSelMaxRows || depth < 0 || hq <= 0 || hq % p->h_kv() != 0) {
         return -1;
     }
-    return fnkv::plan_sparse(*p, depth, T, hq / p->h_kv()).bytes;
+    return fnkv::plan_sparse(*p, depth + T - 1, T, hq / p->h_kv()).bytes;
 }
 
 int fnkv_attn_sparse(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_t T, int32_t layer, int32_t hq,

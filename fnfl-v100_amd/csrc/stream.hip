@@ -461,16 +461,15 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
         qv[e] = *reinterpret_cast<const u32x4 *>(
             a.q + ((int64_t(s) * a.T + t_row) * a.hq + int64_t(kvh) * a.G + row % a.G) * kHeadDim + b * kQK + 8 * qg);
     }
-    split_src<false> src;
-    src.template init<64 * WAVES>(a, table, split, begin, ctx < begin + a.split_tokens ? ctx : begin + a.split_tokens,
-                                  lane, smem, nullptr, ctx);
+    split_src src;
+    src.init(a, table, split, begin, ctx < begin + a.split_tokens ? ctx : begin + a.split_tokens, lane, ctx);
     if (a.ctx_dev != nullptr) {
-        ctx = seq_ctx<false>(a, s);
+        ctx = seq_ctx(a, s);
         src.recount(ctx);
     }
     const int64_t end = ctx < begin + a.split_tokens ? ctx : begin + a.split_tokens;
     FNKV_STAMP(6);
-    if (refused<false>(a, s, ctx, sp, kvh)) {
+    if (refused(a, s, ctx, sp, kvh)) {
         return;
     }
     const bool unmapped = src.guard_unmapped(lane);

@@ -236,9 +236,10 @@ int64_t fnkv_qsa_workspace_bytes(const fnkv_pool * pool, int64_t depth, int32_t 
  * 1e-5 normalized bound, qa2_test.cpp:58), and each (row, head) is finished with its gate: out = o / (1 + exp(-gate)) in F32 with its int8 activation format.
  * qfull: F32 [T][hq][512] (each head's q, then its gate); kv_k, kv_v: F32 [T][h_kv][256]; q_norm, k_norm: F32 [256];
  * out: F32 [T][hq][256]; codes: int8 [T][hq 256]; scales: F32 [T][hq 8][2]; q_f32, k_f32 (optional): the F32 q
- * [T][hq][256] and k [T][h_kv][256] after the norm and rope. Three launches in stream order: the prepare (which
+ * [T][hq][256] and k [T][h_kv][256] after the norm and rope. Up to three launches in stream order: the prepare (which
  * writes the new cells), the attention (each row its own splits), the gated merge; at most 16 query heads a KV head:
- * two (the attention forms each row's query heads and writes the new cells itself, bitwise the same outputs).
+ * no prepare launch (the attention forms each row's query heads and writes the new cells itself, bitwise the same
+ * outputs); rows that fit one split: no merge.
  * hq / h_kv <= FNKV_MAX_ROWS. */
 int fnkv_qsa_attend(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_t T, int32_t layer, int32_t hq,
                     const float * qfull, const float * kv_k, const float * kv_v, const float * q_norm,

@@ -1,0 +1,78 @@
+"""The sparse launch's virtual tiles (eight selected 4-cell blocks each, four a split) at the sizes where they can go
+wrong: rows of one entry, of a full tile less, exactly and plus one entry, of a full split (32 entries) around its edges
+and of the most entries (512 blocks with each tail), an ID repeated in a body, selections whose blocks share a pool tile
+in every arrangement, and prompts whose row count sits at the edges of the rule that splits rows. Each against the
+oracle's fp64 attention over the selected cells (max-abs 2e-3, test_gpu_sparse.py's and test_gpu_qsp.py's bound)."""
+import numpy as np
+import pytest
+
+import cases
+import fnkv
+import oracle as O
+import test_gpu_qsp as qsp
+import test_gpu_sparse as sparse
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+TOL = 2e-3
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+@pytest.mark.parametrize("fmt", [fnkv.FMT_Q8_0, fnkv.FMT_KV8])
+@pytest.mark.parametrize("depth", [1, 3, 4, 26, 30, 31, 34, 126, 127, 130, 254, 2042, 2046, 2047, 2049, 5002])
+def test_entries_at_tile_and_split_edges(depth, fmt):
+    pool, got, ref, _ = sparse.sparse_case(depth, 1, seed=depth + 900, fmt=fmt)
+    assert np.isfinite(got).all()
+    assert cases.out_err(got, ref) <= TOL
+
+
+@pytest.mark.parametrize("T", [1, 4])
+def test_repeated_ids_count_once(T):
+    # every row's sixth and seventh entries repeat its fifth, the last repeats the one before it
+    depth = 6001
+    words, offs, _ = O.qsa_body(depth, T, seed=61)
+    w = words.view(np.int32).copy()
+    cells = []
+    for t in range(T):
+        o, n_vis = offs[t] // 4, (depth + t + 1) // 4
+        ids = w[o + 2:o + 2 + w[o]]
+        ids[5] = ids[6] = ids[4]
+        ids[-1] = ids[-2]
+        b = np.unique(ids).astype(np.int64)
+        cells.append(np.concatenate([(4 * b[:, None] + np.arange(4)).reshape(-1), np.arange(4 * n_vis, depth + t + 1)]))
+    pool, got, ref, _ = sparse.sparse_case(depth, T, seed=61, body=(w.view(np.uint32), offs, cells))
+    assert cases.out_err(got, ref) <= TOL
+
+
+@pytest.mark.parametrize("blocks_of_tile", [[0], [7], [0, 4], [3, 4], [1, 2, 3], [0, 2, 4, 6], list(range(8))])
+def test_blocks_that_share_a_pool_tile(blocks_of_tile):
+    # 512 blocks, the same ones of every tile (the last tiles fill up to 512)
+    depth, T = 20000, 1
+    n_vis = (depth + 1) // 4
+    tiles = np.arange(n_vis // 8 - 2)[-(512 // len(blocks_of_tile)):]
+    b = (8 * tiles[:, None] + np.array(blocks_of_tile)).reshape(-1)
+    b = np.unique(np.concatenate([np.setdiff1d(np.arange(n_vis), b)[:512 - b.size], b]))
+    tail = np.arange(4 * n_vis, depth + 1)
+    words = np.concatenate([[512, tail.size], b, tail]).astype(np.uint32)
+    cells = [np.concatenate([(4 * b[:, None] + np.arange(4)).reshape(-1), tail])]
+    pool, got, ref, _ = sparse.sparse_case(depth, T, seed=71,
+                                           body=(words, np.array([0, 4 * words.size], np.int32), cells))
+    assert cases.out_err(got, ref) <= TOL
+
+
+# pairs (row, 16-head tile of a KV head) a launch: 17 splits a row up to 30, one split from 257 on (256 CUs, two
+# workgroups each)
+@pytest.mark.parametrize("rows,hq,h_kv", [(6, 12, 1), (30, 12, 1), (31, 12, 1), (129, 16, 2), (256, 12, 1), (257, 12, 1),
+                                          (70, 40, 2)])
+def test_prompt_rows_at_the_split_rule(rows, hq, h_kv):
+    o16, o32, err, ref = qsp.run_attend(3000, rows, hq, h_kv, seed=rows + hq)
+    assert err == 0 and np.isfinite(o32).all()
+    assert float(np.abs(o32.astype(np.float64) - ref).max()) <= TOL
+    assert np.array_equal(o16.view(np.uint16), o32.astype(np.float16).view(np.uint16))
