@@ -13,7 +13,8 @@
 //   * A workgroup (8 waves, two a SIMD, so one wave's matrix-core work overlaps the other's VALU work) owns 256 query
 //     rows (256 / G query tokens x the G heads of one KV head); each wave owns two 16-row tiles, so each operand
 //     read from LDS feeds two MFMAs. Its waves walk the key tiles (32 tokens) of the workgroup's key split in order;
-//     the splits (blockIdx.z) fill the device when the row blocks alone do not, and a merge kernel folds them.
+//     the splits fill the device when the row blocks alone do not (plan_prefill), and a merge kernel folds them. Only
+//     workgroups whose row block sees their split are launched.
 //   * Each tile's codes go from HBM straight into the registers of the wave that converts them (wave w: K chunk w
 //     and V chunk w, a tile ahead), its scales chunk into a small LDS ring; every wave writes its two chunks as fp16
 //     operand planes (K codes, V codes; double-buffered: tile k + 1's while tile k is computed), and four waves
@@ -22,8 +23,18 @@
 //     O^T += V^T P^T (two a 16-value tile and row tile: the codes against (P x V scale) hi and lo). Against
 //     dequantized hi + lo K and V planes this halves the operand bytes each wave reads from LDS and cuts the MFMAs a
 //     wave and tile from 159 to 96.
+//   * The scores and PV run one block behind themselves: a block's scale FMAs stand behind the next block's MFMAs
+//     (four to one), a block's P x V-scale products among the previous block's. In program order a wave that waits
+//     for a busy matrix core cannot reach its own VALU work, and the two waves of a SIMD, aligned by the tile's
+//     barrier, are in the same phase. Half of q's operands sit in LDS to make the registers for it.
 //   * The softmax (base 2, the running max moved lazily) runs on the S^T registers as in the decode kernel; P feeds
 //     the PV MFMA in place.
+// What bounds it: a long launch, the chip's power. 2,048 rows over 133,120 cells take 7.10 -> 6.86-6.95 ms with the
+// interleaving although its cycles fall further: the matrix cores' overlap with the VALU rises and the clock falls from
+// 2.31 to ~2.1 GHz (a 32x32x16 form: 12.5% fewer cycles at 1.94 GHz, 7.14-7.25 ms). Its three MFMA passes (scores, P hi,
+// P lo) run at 960 TFLOP/s where a large fp16 GEMM reaches 1,070-1,130 on this card. A short one is bound by its tiles'
+// latency and the partials: 517 rows over 3,001 cells 102 -> 78 us with the append (9 of it the interleaving, 15 the
+// splits), a 2,048-cell prompt's own 2,048 rows 152 -> 113 us, 16 rows at 131,088 cells 280 -> 143 us.
 #include "../../include/fnkv.h"
 #include "common.h"
 #include "layout.h"
@@ -63,7 +74,13 @@ constexpr int32_t kPfKscOff = 2 * kPfPlane;
 constexpr int32_t kPfSet = kPfKscOff + kPfKsc;       // a tile's planes: K codes, V codes, K scales
 constexpr int32_t kPfScaleRing = 4;                  // tiles' scale chunks (K then V scales, 1 KiB), a ring
 constexpr int32_t kPfPages = 2048;                   // the split's page table entries held in LDS (a split <= 512 K cells)
-constexpr int32_t kPfLds = 2 * kPfSet + kPfScaleRing * 1024 + kPfPages * 4; // planes double-buffered, ring, pages
+constexpr int32_t kPfRegBlocks = 4;                  // q's blocks held in registers; the others' operands sit in LDS
+constexpr int32_t kPfQWave = (kBlocks - kPfRegBlocks) * kPfNT * 1024; // a wave's: [block][row tile][lane] 16 B
+constexpr int32_t kPfQOff = 2 * kPfSet + kPfScaleRing * 1024 + kPfPages * 4;
+constexpr int32_t kPfLds = kPfQOff + kPfWaves * kPfQWave; // planes double-buffered, ring, pages, q
+static_assert(kPfLds <= 160 * 1024, "LDS");
+// instruction groups of __builtin_amdgcn_sched_group_barrier
+constexpr int kSchedValu = 0x2, kSchedMfma = 0x8, kSchedDsRead = 0x100;
 constexpr float kPfNegInf = -__builtin_inff();
 constexpr float kPfLazyLog2 = 6.0f; // the running max moves only past this margin
 
@@ -71,12 +88,12 @@ struct pf_args {
     pool_view pv;
     const uint16_t * q; // fp16 [rows][hq][256]
     uint16_t * out;     // fp16 [rows][hq][256]
-    float * po;         // split partials (n_split > 1): acc [split][h_kv][row blocks * kPfRows][256]
-    float * pml;        // ... and (m, l) [split][h_kv][row blocks * kPfRows][2]
+    float * po;         // split partials (n_split > 1): acc [split][h_kv][rows G][256], of the splits a row block reaches
+    float * pml;        // ... and (m, l) [split][h_kv][rows G][2]
     float c2;           // scale * log2(e)
     int64_t ctx;        // cells of the sequence (the chunk included)
     int32_t rows, G, hq, layer, slot;
-    int32_t n_split, split_tiles; // key tiles split over blockIdx.z: split z takes tiles z * split_tiles ..
+    int32_t row_blocks, n_split, split_tiles; // split z takes the key tiles z * split_tiles ..
 #ifdef FNKV_TIMING
     uint64_t * ts; // per wave: phase cycle sums (instrumented builds only)
 #endif
@@ -95,15 +112,38 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
     const int32_t lane = static_cast<int32_t>(threadIdx.x) & 63;
     const int32_t wave = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x) >> 6);
     const int32_t j = lane & 15, qg = lane >> 4;
-    const int32_t kvh = static_cast<int32_t>(blockIdx.y);
+    const int32_t h_kv = a.pv.h_kv;
     const int32_t tok_per_wg = kPfRows / a.G;
-    const int32_t t_first = static_cast<int32_t>(blockIdx.x) * tok_per_wg;
     const int64_t pos_first = a.ctx - a.rows; // position of query token 0
+    // workgroup -> (KV head, row block, split), split by split over the row blocks that see it (a block sees the keys up
+    // to its last query's): the workgroups without keys are not launched, so the others spread evenly over the XCDs
+    const int32_t kvh = static_cast<int32_t>(blockIdx.x) % h_kv;
+    int32_t blk = static_cast<int32_t>(blockIdx.x) / h_kv, z;
+    const int64_t split_keys = int64_t(a.split_tiles) * kTileTokens;
+    {
+        const int64_t seen0 = pos_first + min(a.rows, tok_per_wg); // keys block 0 sees: its splits are every block's
+        const int32_t full = static_cast<int32_t>((seen0 + split_keys - 1) / split_keys);
+        if (blk < full * a.row_blocks) {
+            z = blk / a.row_blocks;
+            blk %= a.row_blocks;
+        } else {
+            blk -= full * a.row_blocks;
+            for (z = full; z < a.n_split; ++z) {
+                const int32_t first = static_cast<int32_t>((z * split_keys - pos_first) / tok_per_wg);
+                if (blk < a.row_blocks - first) {
+                    blk += first;
+                    break;
+                }
+                blk -= a.row_blocks - first;
+            }
+        }
+    }
+    const int32_t t_first = blk * tok_per_wg;
     const int32_t t_last = min(a.rows, t_first + tok_per_wg) - 1;
     const int64_t key_end = pos_first + t_last + 1; // keys the block's last query sees
     const int32_t n_tiles_all = static_cast<int32_t>((key_end + kTileTokens - 1) / kTileTokens);
     // this workgroup's key tiles: its split's share of those the block's queries see
-    const int32_t ts0 = static_cast<int32_t>(blockIdx.z) * a.split_tiles;
+    const int32_t ts0 = z * a.split_tiles;
     const int32_t n_tiles = max(0, min(n_tiles_all, ts0 + a.split_tiles) - ts0);
 
     const pool_view & pv = a.pv;
@@ -144,7 +184,8 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
     }
 
     // Q operands (B of S^T = K Q^T) of this wave's two row tiles, and each row's causal limit
-    half8 qop[kPfNT][kBlocks];
+    half8 qreg[kPfNT][kPfRegBlocks];
+    uint8_t * const qlds = smem + kPfQOff + wave * kPfQWave + lane * 16;
     int32_t lim[kPfNT]; // each row's last visible cell, relative to the split's first
 #pragma unroll
     for (int nt = 0; nt < kPfNT; ++nt) {
@@ -159,9 +200,17 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
             if (real) {
                 v = *reinterpret_cast<const u32x4 *>(qrow + b * kQK + 8 * qg);
             }
-            qop[nt][b] = __builtin_bit_cast(half8, v);
+            if (b < kPfRegBlocks) {
+                qreg[nt][b < kPfRegBlocks ? b : 0] = __builtin_bit_cast(half8, v);
+            } else {
+                *reinterpret_cast<u32x4 *>(qlds + ((b - kPfRegBlocks) * kPfNT + nt) * 1024) = v;
+            }
         }
     }
+    auto q_at = [&](int nt, int b) {
+        return b < kPfRegBlocks ? qreg[nt][b < kPfRegBlocks ? b : 0]
+                                : *reinterpret_cast<const half8 *>(qlds + ((b - kPfRegBlocks) * kPfNT + nt) * 1024);
+    };
     floatx4 acc[kPfNT][16];
     float m_run[kPfNT], l_run[kPfNT];
 #pragma unroll
@@ -213,36 +262,71 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
             sc[nt][0] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
             sc[nt][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
         }
-        // S^T block by block: the block's MFMA on the exact codes, then its K scale (the lane's four tokens) by one
-        // FMA a score; the next block's operands are read from LDS while this block's MFMAs run
-        auto kc_at = [&](int hb) { return *reinterpret_cast<const half8 *>(pl + (hb * 64 + lane) * 16); };
-        auto ks_at = [&](int hb) { return *reinterpret_cast<const half4v *>(pl + kPfKscOff + (hb * 4 + qg) * 8); };
-        half8 kc_next = kc_at(0);
-        half4v ks_next = ks_at(0);
+        {
+            auto kc_at = [&](int b, int h) {
+                return *reinterpret_cast<const half8 *>(pl + ((h * kBlocks + b) * 64 + lane) * 16);
+            };
+            auto ks_at = [&](int b, int h) {
+                return *reinterpret_cast<const half4v *>(pl + kPfKscOff + ((h * kBlocks + b) * 4 + qg) * 8);
+            };
+            floatx4 t[2][kPfNT][2];
+            half8 kc[2], kq[kPfNT];
+            half4v ks[2];
+            auto operands = [&](int b) {
+                kc[0] = kc_at(b, 0);
+                kc[1] = kc_at(b, 1);
 #pragma unroll
-        for (int hb = 0; hb < 2 * kBlocks; ++hb) {
-            const int h = hb / kBlocks, b = hb % kBlocks;
-            const half8 kc = kc_next;
-            const half4v ks = ks_next;
-            if (hb + 1 < 2 * kBlocks) {
-                kc_next = kc_at(hb + 1);
-                ks_next = ks_at(hb + 1);
-            }
-            floatx4 t[kPfNT];
-#pragma unroll
-            for (int nt = 0; nt < kPfNT; ++nt) {
-                t[nt] = mfma16(kc, qop[nt][b], floatx4{0.0f, 0.0f, 0.0f, 0.0f});
-            }
-#pragma unroll
-            for (int nt = 0; nt < kPfNT; ++nt) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    sc[nt][h][r] = __builtin_fmaf(static_cast<float>(ks[r]), t[nt][r], sc[nt][h][r]);
+                for (int nt = 0; nt < kPfNT; ++nt) {
+                    kq[nt] = q_at(nt, b);
                 }
-                __asm__ volatile("" : "+v"(sc[nt][h]));
-            }
-            if (hb & 1) {
-                __builtin_amdgcn_sched_barrier(0); // two blocks' products live at a time
+            };
+            auto scores = [&](int b) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) { // (consecutive MFMAs share their A operand: measured to cost least power)
+                    const int h = m >> 1, nt = m & 1;
+                    t[b & 1][nt][h] = mfma16(kc[h], kq[nt], floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+                }
+            };
+            operands(0);
+            ks[0] = ks_at(0, 0);
+            ks[1] = ks_at(0, 1);
+            scores(0);
+            operands(1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                const half4v ks0 = ks[0], ks1 = ks[1];
+                if (b + 1 < kBlocks) {
+                    scores(b + 1);
+                    ks[0] = ks_at(b + 1, 0);
+                    ks[1] = ks_at(b + 1, 1);
+                }
+                if (b + 2 < kBlocks) {
+                    operands(b + 2);
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                    for (int nt = 0; nt < kPfNT; ++nt) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            sc[nt][h][r] = __builtin_fmaf(static_cast<float>(h == 0 ? ks0[r] : ks1[r]),
+                                                          t[b & 1][nt][h][r], sc[nt][h][r]);
+                        }
+                        __asm__ volatile("" : "+v"(sc[nt][h]));
+                    }
+                }
+                if (b + 1 < kBlocks) { // each MFMA of block b + 1 with four of block b's FMAs behind it
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+                        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+                        if (m == 3) {
+                            __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 8, 0);
+                        }
+                        __builtin_amdgcn_sched_group_barrier(kSchedValu, 4, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
 #ifdef FNKV_TIMING
@@ -309,23 +393,42 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
         // O^T += V^T P^T block by block: P times the block's V scales (this lane's 8 tokens) as hi + lo fp16 (to
         // ~2^-19), against the exact codes
         const uint8_t * rgv = ring(ti) + 512 + qg * 128;
-#pragma unroll
-        for (int b = 0; b < kBlocks; ++b) {
-            const half8 v0 = *reinterpret_cast<const half8 *>(pl + kPfPlane + ((2 * b) * 64 + lane) * 16);
-            const half8 v1 = *reinterpret_cast<const half8 *>(pl + kPfPlane + ((2 * b + 1) * 64 + lane) * 16);
-            const half8 vsb = *reinterpret_cast<const half8 *>(rgv + b * 16);
+        half8 hi[2][kPfNT], lo[2][kPfNT], vs, v[2];
+        auto products = [&](int b) {
 #pragma unroll
             for (int nt = 0; nt < kPfNT; ++nt) {
-                half8 hi, lo;
-                scale_hilo_pk(ph[nt], plo[nt], vsb, hi, lo);
-                acc[nt][2 * b] = mfma16(v0, hi, acc[nt][2 * b]);
-                acc[nt][2 * b + 1] = mfma16(v1, hi, acc[nt][2 * b + 1]);
-                acc[nt][2 * b] = mfma16(v0, lo, acc[nt][2 * b]);
-                acc[nt][2 * b + 1] = mfma16(v1, lo, acc[nt][2 * b + 1]);
+                scale_hilo_pk(ph[nt], plo[nt], vs, hi[b & 1][nt], lo[b & 1][nt]);
             }
-            if (b & 1) {
-                __builtin_amdgcn_sched_barrier(0); // two blocks' operands live at a time
+        };
+        auto codes_at = [&](int b, int m) {
+            return *reinterpret_cast<const half8 *>(pl + kPfPlane + ((2 * b + m) * 64 + lane) * 16);
+        };
+        vs = *reinterpret_cast<const half8 *>(rgv);
+        products(0);
+        vs = *reinterpret_cast<const half8 *>(rgv + 16);
+        v[0] = codes_at(0, 0);
+        v[1] = codes_at(0, 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) {
+            const half8 v0 = v[0], v1 = v[1];
+            auto pv = [&](int m, half8 va) { // consecutive MFMAs share their A operand
+                acc[0][2 * b + m] = mfma16(va, hi[b & 1][0], acc[0][2 * b + m]);
+                acc[1][2 * b + m] = mfma16(va, hi[b & 1][1], acc[1][2 * b + m]);
+                acc[0][2 * b + m] = mfma16(va, lo[b & 1][0], acc[0][2 * b + m]);
+                acc[1][2 * b + m] = mfma16(va, lo[b & 1][1], acc[1][2 * b + m]);
+            };
+            pv(0, v0);
+            if (b + 1 < kBlocks) {
+                products(b + 1);
+                v[0] = codes_at(b + 1, 0);
+                v[1] = codes_at(b + 1, 1);
             }
+            pv(1, v1);
+            if (b + 2 < kBlocks) {
+                vs = *reinterpret_cast<const half8 *>(rgv + (b + 2) * 16);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
 
@@ -362,7 +465,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
     wait_vmcnt<0>();
 #ifdef FNKV_TIMING
     if (lane == 0 && a.ts != nullptr) {
-        const int64_t wg = (int64_t(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+        const int64_t wg = blockIdx.x;
         for (int i = 0; i < 8; ++i) {
             a.ts[(wg * kPfWaves + wave) * 8 + i] = pf_ph[i];
         }
@@ -371,12 +474,15 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
 
     // ---- one split: normalise and write; several: the unnormalised partial (acc, m, l) for the merge ----
     if (a.n_split > 1) {
-        const int64_t prow0 = (int64_t(blockIdx.z) * gridDim.y + kvh) * (int64_t(gridDim.x) * kPfRows) +
-                              int64_t(blockIdx.x) * kPfRows;
+        const int64_t n_rows = int64_t(a.rows) * a.G;
 #pragma unroll
         for (int nt = 0; nt < kPfNT; ++nt) {
             const float l = rows_sum(l_run[nt]);
-            const int64_t prow = prow0 + (wave * kPfNT + nt) * 16 + j;
+            const int64_t R = int64_t(blk) * kPfRows + (wave * kPfNT + nt) * 16 + j;
+            if (R >= n_rows) {
+                continue;
+            }
+            const int64_t prow = (int64_t(z) * h_kv + kvh) * n_rows + R;
             float * po = a.po + prow * kHeadDim + 4 * qg;
 #pragma unroll
             for (int m = 0; m < 16; ++m) {
@@ -411,39 +517,58 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
 }
 
 // Folds the splits' partials of each (query token, head): M = max m_z, L = sum l_z 2^(m_z - M), O = sum acc_z
-// 2^(m_z - M) / L, in split order. A thread takes 4 values of one row; 64 threads a row.
-__global__ __launch_bounds__(256) void prefill_merge_kernel(pf_args a, int32_t rows_pad) {
-    const int32_t tid = static_cast<int32_t>(threadIdx.x);
-    const int64_t item = int64_t(blockIdx.x) * 4 + (tid >> 6); // (kvh, row) over h_kv x rows_pad
-    const int32_t c4 = (tid & 63) * 4;
+// 2^(m_z - M) / L over the splits the token's row block reaches. A wave takes a row's splits g, g + GRP, ... in order
+// with a running max (4 values a lane, four splits' loads in flight); the GRP waves of a row then fold in order in LDS.
+// A workgroup of 4 waves holds 4 / GRP rows.
+template <int GRP> __global__ __launch_bounds__(256) void prefill_merge_kernel(pf_args a) {
+    __shared__ floatx4 sA[4][64];
+    __shared__ float2 sML[4];
+    const int32_t wave = static_cast<int32_t>(threadIdx.x) >> 6, lane = static_cast<int32_t>(threadIdx.x) & 63;
+    const int32_t g = wave % GRP;
+    const int64_t n_rows = int64_t(a.rows) * a.G;
     const int32_t h_kv = a.pv.h_kv;
-    if (item >= int64_t(h_kv) * rows_pad) {
-        return;
+    const int64_t item = int64_t(blockIdx.x) * (4 / GRP) + wave / GRP; // (kvh, row)
+    if (item >= h_kv * n_rows) {
+        return; // (a workgroup of one row, GRP = 4, never leaves in part)
     }
-    const int32_t kvh = static_cast<int32_t>(item / rows_pad);
-    const int32_t R = static_cast<int32_t>(item % rows_pad);
+    const int64_t kvh = item / n_rows, R = item % n_rows;
+    const int32_t t = static_cast<int32_t>(R / a.G);
     const int32_t tok_per_wg = kPfRows / a.G;
-    const int32_t blk = R / kPfRows, r = R % kPfRows;
-    const int32_t t = blk * tok_per_wg + r / a.G;
-    if (t >= a.rows) {
-        return;
-    }
-    float M = kPfNegInf;
-    for (int32_t z = 0; z < a.n_split; ++z) {
-        M = fmaxf(M, a.pml[((int64_t(z) * h_kv + kvh) * rows_pad + R) * 2]);
-    }
-    const float M_use = M == kPfNegInf ? 0.0f : M;
-    float L = 0.0f;
+    const int32_t t_last = min(a.rows, (t / tok_per_wg + 1) * tok_per_wg) - 1; // the row block's last token
+    const int64_t tiles = (a.ctx - a.rows + t_last + kTileTokens) / kTileTokens;
+    const int32_t n = static_cast<int32_t>(min(int64_t(a.n_split), (tiles + a.split_tiles - 1) / a.split_tiles));
+    float M = kPfNegInf, L = 0.0f;
     floatx4 A = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int32_t z = 0; z < a.n_split; ++z) {
-        const int64_t prow = (int64_t(z) * h_kv + kvh) * rows_pad + R;
+    auto fold = [](float & m0, float & l0, floatx4 & A0, float m1, float l1, floatx4 A1) {
+        const float mn = fmaxf(m0, m1);
+        const float mu = mn == kPfNegInf ? 0.0f : mn;
+        const float f0 = __builtin_amdgcn_exp2f(m0 - mu), f1 = __builtin_amdgcn_exp2f(m1 - mu);
+        A0 = A0 * f0 + A1 * f1;
+        l0 = __builtin_fmaf(l0, f0, l1 * f1);
+        m0 = mn;
+    };
+#pragma unroll 4
+    for (int32_t z = g; z < n; z += GRP) {
+        const int64_t prow = (int64_t(z) * h_kv + kvh) * n_rows + R;
         const float2 ml = *reinterpret_cast<const float2 *>(a.pml + prow * 2);
-        const float f = __builtin_amdgcn_exp2f(ml.x - M_use);
-        L = __builtin_fmaf(ml.y, f, L);
-        A += *reinterpret_cast<const floatx4 *>(a.po + prow * kHeadDim + c4) * f;
+        fold(M, L, A, ml.x, ml.y, *reinterpret_cast<const floatx4 *>(a.po + prow * kHeadDim + lane * 4));
+    }
+    if constexpr (GRP > 1) {
+        sA[wave][lane] = A;
+        if (lane == 0) {
+            sML[wave] = float2{M, L};
+        }
+        __syncthreads();
+        if (g != 0) {
+            return;
+        }
+#pragma unroll
+        for (int32_t w = 1; w < GRP; ++w) {
+            fold(M, L, A, sML[wave + w].x, sML[wave + w].y, sA[wave + w][lane]);
+        }
     }
     const float inv = 1.0f / L;
-    uint16_t * o = a.out + (int64_t(t) * a.hq + int64_t(kvh) * a.G + r % a.G) * kHeadDim + c4;
+    uint16_t * o = a.out + (int64_t(t) * a.hq + kvh * a.G + R % a.G) * kHeadDim + lane * 4;
     uint2 pk;
     pk.x = uint32_t(__half_as_ushort(__float2half_rn(A[0] * inv))) |
            (uint32_t(__half_as_ushort(__float2half_rn(A[1] * inv))) << 16);
@@ -452,29 +577,57 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(pf_args a, int32_t r
     *reinterpret_cast<uint2 *>(o) = pk;
 }
 
-// The launch shape: row blocks of kPfRows rows, and the key split that fills the device (a split keeps at least 16
-// tiles); the workspace the splits' partials need (0 for one split).
+// The launch shape: row blocks of kPfRows rows, and the key split with the least time: the rounds of one workgroup a CU
+// (of the workgroups whose block sees their split: a causal chunk's first blocks see few tiles) times a workgroup's tiles
+// (3.4 us each) plus a fixed cost of kPfFixed tiles (the first tile's round trips, q, the partial's write), plus, for
+// more than one split, the merge launch (one tile's time) and the partials' way through memory (written and read at
+// about 4 TB/s: 13.6 MB a tile's time).
 struct pf_plan {
-    int32_t row_blocks = 0, n_split = 1, split_tiles = 0, rows_pad = 0;
+    int32_t row_blocks = 0, n_split = 1, split_tiles = 0;
+    int64_t wgs = 0; // workgroups: each block's splits
     int64_t ws_bytes = 0;
 };
+constexpr int32_t kPfFixed = 5;
+constexpr int32_t kPfMaxSplit = 256;
 pf_plan plan_prefill(const kv_pool & p, int64_t ctx, int32_t rows, int32_t G) {
     pf_plan pl;
     const int32_t tok_per_wg = kPfRows / G;
     pl.row_blocks = (rows + tok_per_wg - 1) / tok_per_wg;
-    pl.rows_pad = pl.row_blocks * kPfRows;
-    const int32_t max_tiles = static_cast<int32_t>((ctx + kTileTokens - 1) / kTileTokens);
-    const int32_t base = pl.row_blocks * p.h_kv();
-    const int32_t cus = device_cus(p.device());
-    int32_t ns = (cus + base - 1) / base;
-    ns = std::min(ns, std::max(1, max_tiles / 16));
+    const int64_t max_tiles = (ctx + kTileTokens - 1) / kTileTokens;
+    const int64_t cus = device_cus(p.device());
+    const int64_t split_bytes = int64_t(p.h_kv()) * rows * G * (kHeadDim + 2) * 4; // one split's partials
     // a split's pages fit the kernel's LDS copy of the table
-    ns = std::max(ns, (max_tiles + kPfPages * kTilesPerPage - kTilesPerPage - 1) / (kPfPages * kTilesPerPage - kTilesPerPage));
-    ns = std::min(ns, 64);
-    pl.n_split = std::max(1, ns);
-    pl.split_tiles = (max_tiles + pl.n_split - 1) / pl.n_split;
+    const int64_t page_tiles = kPfPages * kTilesPerPage - kTilesPerPage;
+    const int64_t least = std::max<int64_t>(1, (max_tiles + page_tiles - 1) / page_tiles);
+    const int64_t most = std::max(least, std::min<int64_t>(kPfMaxSplit, max_tiles));
+    auto workgroups = [&](int64_t size) { // with tiles, at splits of `size` tiles
+        int64_t n = 0;
+        for (int32_t b = 0; b < pl.row_blocks; ++b) {
+            const int64_t seen = ctx - rows + std::min(rows, (b + 1) * tok_per_wg); // keys the block's last query sees
+            n += (seen + size * kTileTokens - 1) / (size * kTileTokens);
+        }
+        return n * p.h_kv();
+    };
+    double best = 0.0;
+    for (int64_t ns = least; ns <= most; ++ns) {
+        const int64_t size = (max_tiles + ns - 1) / ns;
+        const int64_t wgs = workgroups(size);
+        const int64_t rounds = (wgs + cus - 1) / cus;
+        if (ns > least && rounds > 2) {
+            break; // more rounds only add fixed cost and partials
+        }
+        const double bytes = double(split_bytes) * double(wgs) / double(pl.row_blocks * p.h_kv());
+        const double cost = double(rounds) * double(size + kPfFixed) + (ns > 1 ? 1.0 + 2.0 * bytes / 13.6e6 : 0.0);
+        if (ns == least || cost < best) {
+            best = cost;
+            pl.n_split = static_cast<int32_t>(ns);
+        }
+    }
+    pl.split_tiles = static_cast<int32_t>((max_tiles + pl.n_split - 1) / pl.n_split);
+    pl.n_split = static_cast<int32_t>((max_tiles + pl.split_tiles - 1) / pl.split_tiles); // no empty last split
+    pl.wgs = workgroups(pl.split_tiles);
     if (pl.n_split > 1) {
-        pl.ws_bytes = int64_t(pl.n_split) * p.h_kv() * pl.rows_pad * (kHeadDim + 2) * 4;
+        pl.ws_bytes = pl.n_split * split_bytes;
     }
     return pl;
 }
@@ -528,14 +681,16 @@ int fnkv_attn_prefill(const fnkv_pool * pool, int32_t slot, int32_t layer, int64
         // no (or too small a) workspace: one split, written directly
         pl.n_split = 1;
         pl.split_tiles = static_cast<int32_t>((ctx + fnkv::kTileTokens - 1) / fnkv::kTileTokens);
+        pl.wgs = int64_t(pl.row_blocks) * p->h_kv();
     }
+    a.row_blocks = pl.row_blocks;
     a.n_split = pl.n_split;
     a.split_tiles = pl.split_tiles;
 #ifdef FNKV_TIMING
     a.ts = fnkv::timing_buffer();
 #endif
     a.po = static_cast<float *>(ws);
-    a.pml = a.po == nullptr ? nullptr : a.po + int64_t(pl.n_split) * p->h_kv() * pl.rows_pad * fnkv::kHeadDim;
+    a.pml = a.po == nullptr ? nullptr : a.po + int64_t(pl.n_split) * p->h_kv() * rows * G * fnkv::kHeadDim;
     static std::once_flag attr_once[64]; // once per device; a racing first caller waits for it
     const int32_t dev = p->device();
     if (dev >= 0 && dev < 64) {
@@ -549,14 +704,17 @@ int fnkv_attn_prefill(const fnkv_pool * pool, int32_t slot, int32_t layer, int64
             (void)hipSetDevice(cur);
         });
     }
-    const dim3 grid(static_cast<uint32_t>(pl.row_blocks), static_cast<uint32_t>(p->h_kv()),
-                    static_cast<uint32_t>(pl.n_split));
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(fnkv::prefill_kernel, grid, dim3(64 * fnkv::kPfWaves), fnkv::kPfLds, st, a);
+    hipLaunchKernelGGL(fnkv::prefill_kernel, dim3(static_cast<uint32_t>(pl.wgs)), dim3(64 * fnkv::kPfWaves), fnkv::kPfLds, st, a);
     if (pl.n_split > 1) {
-        const int64_t items = int64_t(p->h_kv()) * pl.rows_pad;
-        hipLaunchKernelGGL(fnkv::prefill_merge_kernel, dim3(static_cast<uint32_t>((items + 3) / 4)), dim3(256), 0, st,
-                           a, pl.rows_pad);
+        // a row's splits over four waves from 9 splits on (then the rows are few: a wave's chain of loads is what counts)
+        const int64_t items = int64_t(p->h_kv()) * rows * G;
+        if (pl.n_split > 8) {
+            hipLaunchKernelGGL(fnkv::prefill_merge_kernel<4>, dim3(static_cast<uint32_t>(items)), dim3(256), 0, st, a);
+        } else {
+            hipLaunchKernelGGL(fnkv::prefill_merge_kernel<1>, dim3(static_cast<uint32_t>((items + 3) / 4)), dim3(256), 0,
+                               st, a);
+        }
     }
     if (hipGetLastError() != hipSuccess) {
         set_error("fnkv_attn_prefill: launch failed");

@@ -1,0 +1,51 @@
+"""The chunked prefill's key splits at the shapes where their workgroups' layout changes: causal chunks whose first row
+blocks see fewer splits than the last (none, one or several short), a chunk that starts a prompt, one row block over many
+splits (the four-wave merge), single tiles, last blocks of one token, groups of 1 to 64 query heads. The split launch
+against the launch without a workspace (one split a row block) over every row of outputs filled with NaN first, and the
+chunk's edge rows against the oracle's fp64 attention (max-abs 2e-3; the two launches then agree within twice that)."""
+import numpy as np
+import pytest
+
+import cases
+import fnkv
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+TOL = 2e-3
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+@pytest.mark.parametrize("depth,rows,hq,hkv,fmt", [
+    (0, 1, 16, 2, fnkv.FMT_Q8_0), (0, 32, 16, 2, fnkv.FMT_Q8_0), (31, 1, 16, 2, fnkv.FMT_Q8_0),
+    (0, 33, 16, 1, fnkv.FMT_KV8), (0, 700, 16, 2, fnkv.FMT_Q8_0), (0, 1537, 16, 2, fnkv.FMT_Q8_0),
+    (95, 961, 12, 3, fnkv.FMT_Q8_0), (1000, 513, 16, 2, fnkv.FMT_KV8), (3, 1024, 8, 1, fnkv.FMT_Q8_0),
+    (9000, 16, 16, 2, fnkv.FMT_Q8_0), (9000, 1, 8, 8, fnkv.FMT_Q8_0), (20000, 65, 64, 1, fnkv.FMT_Q8_0),
+    (4000, 257, 1, 1, fnkv.FMT_Q8_0), (6144, 2048, 16, 2, fnkv.FMT_Q8_0)])
+def test_splits_cover_every_row(depth, rows, hq, hkv, fmt):
+    ctx, seed = depth + rows, depth + 3 * rows + hq
+    pool = fnkv.Pool(2, -(-ctx // 256) + 4, 1, hkv, fmt=fmt)
+    cases.scatter_ensure(pool, [0], [ctx], seed, churn=0.3)
+    k16, v16 = cases.kv_rows(seed, ctx, hkv)
+    pool.append(0, 0, 0, torch.from_numpy(k16).cuda(), torch.from_numpy(v16).cuda())
+    q16 = cases.queries(seed, (rows, hq, 256))
+    q = torch.from_numpy(q16).cuda()
+    got, one = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    pool.prefill(0, 0, ctx, q, got)
+    pool.prefill(0, 0, ctx, q, one, ws=False)
+    torch.cuda.synchronize()
+    g, o = got.cpu().numpy().astype(np.float32), one.cpu().numpy().astype(np.float32)
+    assert np.isfinite(g).all() and np.isfinite(o).all()
+    assert cases.out_err(g, o) <= 2 * TOL
+    (_, _, kf), (_, _, vf) = (cases.decoded_kv8 if fmt == fnkv.FMT_KV8 else cases.decoded)(O, k16, v16)
+    check = sorted({0, 1, rows // 3, rows // 2, rows - 2, rows - 1} & set(range(rows)))
+    ref = O.attn_f64(q16.view(np.uint16), kf, vf, ctx, rows=check)
+    assert cases.out_err(got.cpu().numpy()[check], ref) <= TOL
+    assert cases.out_err(one.cpu().numpy()[check], ref) <= TOL
