@@ -299,7 +299,8 @@ __device__ __forceinline__ void append_new_cells(const dec_args & a, const int32
     // sn splits) split tile % sn
     for (int32_t job = wave; job < 2 * a.T; job += WAVES) {
         const int64_t pos = first_new + (job >> 1);
-        const bool mine = sn != 0 ? static_cast<int32_t>((pos >> 5) % sn) == sj : (pos >= begin && pos < end);
+        const bool mine = sn != 0 ? static_cast<uint32_t>(pos >> 5) % static_cast<uint32_t>(sn) == static_cast<uint32_t>(sj)
+                                  : (pos >= begin && pos < end);
         if (!mine) {
             continue;
         }

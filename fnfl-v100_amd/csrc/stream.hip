@@ -20,6 +20,10 @@
 //   * online softmax in base 2 on the S^T registers, which are already the B operand of O^T = V^T P^T; P times the
 //     block's V scale enters the matrix core as fp16 hi + lo (~2^-20 relative); the accumulators O^T (NT x 64
 //     registers) stay in VGPRs (NT <= 2 within a wave's 256);
+//   * both products run as pipelines over the tile's blocks (the next block's VALU work stands between a block's MFMAs,
+//     the LDS reads of the one after ahead of it) and the row tiles' softmax chains side by side: 16 heads on 2 KV
+//     heads, 4,096 cells 14.7 -> 14.3 us a layer, 262,144 cells at 5 rows 93.5 -> 92.0, four sequences of 8K to 64K at
+//     3 rows 37.8 -> 37.5 (the loads bound those: without any of the products a layer still takes 32 us);
 //   * one MFMA pair a tile against the V scales (and a row of ones) gives each row's V bias sums and its l;
 //   * a KV8 pool (group-64 scales, stored at both blocks of a group) takes the KV8 instantiation: a group's two score
 //     MFMAs chain before its one scale FMA, and its P x V-scale products serve both of its blocks;
@@ -61,136 +65,140 @@ template <int NT> struct stream_shape {
     static constexpr int HALF_LOADS = 9;
 };
 
-// S^T = K Q^T of one tile for NT row tiles from the K codes (kb) and the scales chunk (sc) in LDS: sc_out[rt][h][r]
-// is the score (q . k, unscaled) of token 16 h + 4 qg + r against row 16 rt + j. Each 1 KiB chunk of K codes is
-// widened once and feeds the MFMAs of every row tile. KV8: a chunk's two blocks are one 64-value group with one
-// scale, so their two MFMAs chain and the group takes one FMA a score.
+// S^T = K Q^T of one tile for NT row tiles from the K codes (kb) and the scales chunk (sc) in LDS: s_out[rt][h][r]
+// is the score (q . k, unscaled) of token 16 h + 4 qg + r against row 16 rt + j. Each block of K codes is widened once
+// and feeds the MFMAs of every row tile. The blocks run as a pipeline: beside block n + 1's MFMAs stand block n's scale
+// FMAs (one a score), block n + 2's widening and the LDS reads of the operands after those, interleaved with the MFMAs
+// (a wave that waits for a busy matrix core cannot reach VALU work that stands behind it). KV8: a chunk's two blocks are
+// one 64-value group with one scale, so their two MFMAs chain and the group takes one FMA a score.
 template <int NT, bool KV8>
 __device__ __forceinline__ void stream_scores(const uint8_t * kb, const uint8_t * sc, const uint8_t * qs,
                                               const half8 (&sig)[NT], int32_t j, int32_t qg, int32_t lane,
                                               floatx4 (&s_out)[NT][2]) {
     const half8 zero8 = {};
-    // a chunk's operands: its 16 K codes a lane and the row tiles' Q operands of its two blocks; each chunk's are read
-    // from LDS one chunk ahead, while the previous chunk's MFMAs run
+    const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    // block n of the tile's 16 (half n / 8, block n % 8): its codes are words 2 (n & 1), + 1 of chunk n / 2
     auto kw_at = [&](int c) { return *reinterpret_cast<const u32x4 *>(kb + (c >> 2) * 4096 + (c & 3) * 1024 + lane * 16); };
     auto qo_at = [&](int rt, int b) { return *reinterpret_cast<const half8 *>(qs + (rt * kBlocks + b) * 1024 + lane * 16); };
-    u32x4 kw_next = kw_at(0);
-    half8 qo_next[NT][2];
-#pragma unroll
-    for (int rt = 0; rt < NT; ++rt) {
-        qo_next[rt][0] = qo_at(rt, 0);
-        qo_next[rt][1] = qo_at(rt, 1);
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        half8 ks[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            ks[r] = *reinterpret_cast<const half8 *>(sc + (16 * h + 4 * qg + r) * 16);
-        }
-        // the bias term: A = the token row's K scales (lanes qg < 2), B = the row's per-block q sums (hi, lo)
-        const half8 srow = qg < 2 ? *reinterpret_cast<const half8 *>(sc + (16 * h + j) * 16) : zero8;
-        // the scores start from the bias term (-1152 times it) and take each block's term with one FMA a score
-        floatx4 acc_s[NT];
+    u32x4 kw = kw_at(0);
+    half8 ka[2], qo[NT];
+    floatx4 t[2][NT];
+    half8 ks[4];
+    floatx4 acc_s[NT];
+    auto widen = [&](int n) { ka[n & 1] = widen8<false>(kw[2 * (n & 1)], kw[2 * (n & 1) + 1]); };
+    auto load_q = [&](int n) {
 #pragma unroll
         for (int rt = 0; rt < NT; ++rt) {
-            acc_s[rt] = mfma16(srow, sig[rt], floatx4{0.0f, 0.0f, 0.0f, 0.0f}) * -1152.0f;
+            qo[rt] = qo_at(rt, n & 7);
         }
-#pragma unroll
-        for (int ld = 0; ld < 4; ++ld) { // one 1 KiB chunk: blocks 2 ld, 2 ld + 1
-            const int c = 4 * h + ld;
-            const u32x4 kw = kw_next;
-            half8 qo[NT][2];
-#pragma unroll
-            for (int rt = 0; rt < NT; ++rt) {
-                qo[rt][0] = qo_next[rt][0];
-                qo[rt][1] = qo_next[rt][1];
-            }
-            if (c + 1 < 8) {
-                kw_next = kw_at(c + 1);
-#pragma unroll
-                for (int rt = 0; rt < NT; ++rt) {
-                    qo_next[rt][0] = qo_at(rt, 2 * ((c + 1) & 3));
-                    qo_next[rt][1] = qo_at(rt, 2 * ((c + 1) & 3) + 1);
-                }
-            }
-            floatx4 t[NT][2];
-#pragma unroll
-            for (int bb = 0; bb < 2; ++bb) {
-                const half8 ka = widen8<false>(kw[2 * bb], kw[2 * bb + 1]);
-#pragma unroll
-                for (int rt = 0; rt < NT; ++rt) {
-                    if constexpr (KV8) { // the group's second block adds to its first
-                        t[rt][0] = mfma16(ka, qo[rt][bb], bb == 0 ? floatx4{0.0f, 0.0f, 0.0f, 0.0f} : t[rt][0]);
-                    } else {
-                        t[rt][bb] = mfma16(ka, qo[rt][bb], floatx4{0.0f, 0.0f, 0.0f, 0.0f});
-                    }
-                }
-            }
-#pragma unroll
-            for (int bb = 0; bb < (KV8 ? 1 : 2); ++bb) {
-#pragma unroll
-                for (int rt = 0; rt < NT; ++rt) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        acc_s[rt][r] =
-                            __builtin_fmaf(static_cast<float>(ks[r][2 * ld + bb]), t[rt][bb][r], acc_s[rt][r]);
-                    }
-                }
-            }
-            // pin the chunk's FMAs here (the optimizer would otherwise sink them past the later chunks' MFMAs and
-            // keep every chunk's results live at once)
-#pragma unroll
-            for (int rt = 0; rt < NT; ++rt) {
-                __asm__ volatile("" : "+v"(acc_s[rt]));
-            }
-            __builtin_amdgcn_sched_barrier(0); // one chunk's operands live at a time
-        }
+    };
+    auto products = [&](int n) { // t index: the block's, KV8 its group's
+        const int o = KV8 ? (n >> 1) & 1 : n & 1;
 #pragma unroll
         for (int rt = 0; rt < NT; ++rt) {
-            s_out[rt][h] = acc_s[rt];
+            t[o][rt] = mfma16(ka[n & 1], qo[rt], KV8 && (n & 1) == 1 ? t[o][rt] : zero4);
+        }
+    };
+    widen(0);
+    widen(1);
+    load_q(0);
+    kw = kw_at(1);
+    products(0);
+    load_q(1);
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+        const int h = n >> 3, b = n & 7;
+        if (b == 0) { // a half starts: its scales, and the bias term (-1152 times it) that its scores start from
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                ks[r] = *reinterpret_cast<const half8 *>(sc + (16 * h + 4 * qg + r) * 16);
+            }
+            // A = the token row's K scales (lanes qg < 2), B = the row's per-block q sums (hi, lo)
+            const half8 srow = qg < 2 ? *reinterpret_cast<const half8 *>(sc + (16 * h + j) * 16) : zero8;
+#pragma unroll
+            for (int rt = 0; rt < NT; ++rt) {
+                acc_s[rt] = mfma16(srow, sig[rt], zero4) * -1152.0f;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (n + 1 < 16) {
+            products(n + 1);
+        }
+        if (n + 2 < 16) {
+            widen(n + 2);
+            load_q(n + 2);
+        }
+        if ((n & 1) == 1 && n + 3 < 16) {
+            kw = kw_at((n + 3) >> 1);
+        }
+        if (!KV8 || (n & 1) == 1) {
+            const int o = KV8 ? (n >> 1) & 1 : n & 1;
+#pragma unroll
+            for (int rt = 0; rt < NT; ++rt) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    acc_s[rt][r] = __builtin_fmaf(static_cast<float>(ks[r][b]), t[o][rt][r], acc_s[rt][r]);
+                }
+                __asm__ volatile("" : "+v"(acc_s[rt])); // pin the FMAs here: two blocks' products live at a time
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (b == 7) {
+#pragma unroll
+            for (int rt = 0; rt < NT; ++rt) {
+                s_out[rt][h] = acc_s[rt];
+            }
         }
     }
 }
 
-// Online softmax (base 2) of one row tile's tile scores, tokens past lim_rel masked: the row's reference max moves
+// Online softmax (base 2) of the row tiles' tile scores, tokens past lim_rel masked: a row's reference max moves
 // only when the tile's max exceeds it by more than kLazyLog2 (then alpha = 2^(m_old - m_new), else 1), so a weight
 // stays <= 64 and a weight times a V scale stays inside fp16. l is not kept here: the PV step's MFMA against a row
-// of ones sums the weights.
-__device__ __forceinline__ void stream_softmax(const floatx4 (&sc)[2], int32_t lim_rel, float c2, int32_t qg,
-                                               float & m_run, float (&pf)[8], float & alpha) {
-    float raw[8];
-    float mx = kNegInf;
-    if (__all(lim_rel >= 31)) {
+// of ones sums the weights. The row tiles' dependent chains run side by side (no branch between them).
+template <int NT>
+__device__ __forceinline__ void stream_softmax(const floatx4 (&sc)[NT][2], const int32_t (&lim_rel)[NT], float c2,
+                                               int32_t qg, float (&m_run)[NT], half8 (&ph)[NT], half8 (&pl)[NT],
+                                               float (&alpha)[NT]) {
+    float raw[NT][8];
+    bool full = true;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+    for (int rt = 0; rt < NT; ++rt) {
+        full = full && lim_rel[rt] >= 31;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                raw[4 * h + r] = sc[h][r];
-                mx = fmaxf(mx, raw[4 * h + r]);
-            }
+        for (int i = 0; i < 8; ++i) {
+            raw[rt][i] = sc[rt][i >> 2][i & 3];
         }
-    } else {
+    }
+    if (!__all(full)) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int rt = 0; rt < NT; ++rt) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float x = 16 * h + 4 * qg + r <= lim_rel ? sc[h][r] : kNegInf;
-                raw[4 * h + r] = x;
-                mx = fmaxf(mx, x);
+            for (int i = 0; i < 8; ++i) {
+                raw[rt][i] = 16 * (i >> 2) + 4 * qg + (i & 3) <= lim_rel[rt] ? raw[rt][i] : kNegInf;
             }
         }
     }
-    mx = rows_max(mx) * c2;
-    const bool move = mx > m_run + kLazyLog2; // m_run = -inf: any visible score moves it
-    const float m_new = move ? mx : m_run;
-    const float m_use = m_new == kNegInf ? 0.0f : m_new;
-    alpha = move ? __builtin_amdgcn_exp2f(m_run - m_use) : 1.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        pf[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(raw[i], c2, -m_use));
+    for (int rt = 0; rt < NT; ++rt) {
+        float mx = kNegInf;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            mx = fmaxf(mx, raw[rt][i]);
+        }
+        mx = rows_max(mx) * c2;
+        const bool move = mx > m_run[rt] + kLazyLog2; // m_run = -inf: any visible score moves it
+        const float m_new = move ? mx : m_run[rt];
+        const float m_use = m_new == kNegInf ? 0.0f : m_new;
+        alpha[rt] = move ? __builtin_amdgcn_exp2f(m_run[rt] - m_use) : 1.0f;
+        float pf[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            pf[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(raw[rt][i], c2, -m_use));
+        }
+        m_run[rt] = m_new;
+        split_hilo(pf, ph[rt], pl[rt]);
     }
-    m_run = m_new;
 }
 
 // ---- the split-K fold inside the launch ----
@@ -483,7 +491,9 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
         bool owns = false;
         for (int32_t t = 0; t < a.T; ++t) {
             const int64_t pos = ctx - a.T + t;
-            owns |= a.strided ? static_cast<int32_t>((pos >> 5) % src.stride) == src.g0 : (pos >= begin && pos < end);
+            owns |= a.strided ? static_cast<uint32_t>(pos >> 5) % static_cast<uint32_t>(src.stride) ==
+                                    static_cast<uint32_t>(src.g0)
+                              : (pos >= begin && pos < end);
         }
         if (owns) {
             append_new_cells<WAVES>(a, table, s, kvh, ctx, begin, end, src.g0, a.strided ? src.stride : 0, wave,
@@ -588,64 +598,103 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
             FNKV_PHASE(2);
             const int64_t tok0 = src.tok0(st + i * STREAMS);
             half8 ph[NTW], pl[NTW];
+            {
+                int32_t lim_rel[NTW];
+                float alpha[NTW];
+                bool same = true;
 #pragma unroll
-            for (int rt = 0; rt < NTW; ++rt) {
-                const int64_t lr = lim[rt] - tok0;
-                const int32_t lim_rel = lr > 64 ? 64 : static_cast<int32_t>(lr < -1 ? -1 : lr);
-                float pf[8];
-                float alpha;
-                stream_softmax(scv[rt], lim_rel, a.c2, qg, m_run[rt], pf, alpha);
-                if (__any(alpha != 1.0f)) {
-#pragma unroll
-                    for (int b = 0; b < kBlocks; ++b) {
-                        acc[rt][b][0] *= alpha;
-                        acc[rt][b][1] *= alpha;
-                    }
-                    lv[rt] *= alpha;
+                for (int rt = 0; rt < NTW; ++rt) {
+                    const int64_t lr = lim[rt] - tok0;
+                    lim_rel[rt] = lr > 64 ? 64 : static_cast<int32_t>(lr < -1 ? -1 : lr);
                 }
-                split_hilo(pf, ph[rt], pl[rt]);
+                stream_softmax<NTW>(scv, lim_rel, a.c2, qg, m_run, ph, pl, alpha);
+#pragma unroll
+                for (int rt = 0; rt < NTW; ++rt) {
+                    same = same && alpha[rt] == 1.0f;
+                }
+                if (!__all(same)) {
+#pragma unroll
+                    for (int rt = 0; rt < NTW; ++rt) {
+#pragma unroll
+                        for (int b = 0; b < kBlocks; ++b) {
+                            acc[rt][b][0] *= alpha[rt];
+                            acc[rt][b][1] *= alpha[rt];
+                        }
+                        lv[rt] *= alpha[rt];
+                    }
+                }
             }
             FNKV_PHASE(3);
             __builtin_amdgcn_s_setprio(0);
             wait_vmcnt<SH::HALF_LOADS>(); // V(i) has landed (K(i + 1) may be pending)
             FNKV_PHASE(4);
+            // PV as the scores' pipeline: beside block b's MFMAs stand block b + 1's widened codes and P x V-scale
+            // products, and the LDS reads of block b + 2. KV8: a group's two blocks share their scales and products.
+            u32x4 vw = *reinterpret_cast<const u32x4 *>(kb + kVCodes + lane * 16);
+            half8 vs = *reinterpret_cast<const half8 *>(sc + 512 + qg * 128);
+            half8 va[2][2], hi[2][NTW], lo[2][NTW]; // [parity]
+            auto widen_v = [&](int b) {
+                va[b & 1][0] = widen8<false>(vw[0], vw[1]);
+                va[b & 1][1] = widen8<false>(vw[2], vw[3]);
+            };
+            auto set_of = [](int b) { return KV8 ? (b >> 1) & 1 : b & 1; };
+            auto products = [&](int b) {
+#pragma unroll
+                for (int rt = 0; rt < NTW; ++rt) {
+                    scale_hilo_pk(ph[rt], pl[rt], vs, hi[set_of(b)][rt], lo[set_of(b)][rt]);
+                }
+            };
+            auto load_v = [&](int b) {
+                vw = *reinterpret_cast<const u32x4 *>(kb + kVCodes + b * 1024 + lane * 16);
+                if (!KV8 || (b & 1) == 0) {
+                    vs = *reinterpret_cast<const half8 *>(sc + 512 + qg * 128 + b * 16);
+                }
+            };
             // A of the bias MFMAs: lane (block j < 8, qg) holds s_v[token(qg, slot)][j], lanes j = 8 ones (l)
             const half8 sva =
                 j < 8 ? *reinterpret_cast<const half8 *>(sc + 512 + qg * 128 + j * 16) : j == 8 ? ones8 : zero8;
 #pragma unroll
             for (int rt = 0; rt < NTW; ++rt) {
                 lv[rt] = mfma16(sva, ph[rt], lv[rt]);
+            }
+            widen_v(0);
+            products(0);
+#pragma unroll
+            for (int rt = 0; rt < NTW; ++rt) {
                 lv[rt] = mfma16(sva, pl[rt], lv[rt]);
             }
-            // each block's V codes and scales are read from LDS one block ahead
-            u32x4 vw_next = *reinterpret_cast<const u32x4 *>(kb + kVCodes + lane * 16);
-            half8 vs_next = *reinterpret_cast<const half8 *>(sc + 512 + qg * 128);
-            // KV8: a group's two blocks share their scales, so its P x V-scale products serve both
-            half8 phs[NTW], pls[NTW];
+            load_v(1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int b = 0; b < kBlocks; ++b) {
-                const u32x4 vw = vw_next;
-                const half8 vs = vs_next;
                 if (b + 1 < kBlocks) {
-                    vw_next = *reinterpret_cast<const u32x4 *>(kb + kVCodes + (b + 1) * 1024 + lane * 16);
+                    widen_v(b + 1);
                     if (!KV8 || (b & 1) == 1) {
-                        vs_next = *reinterpret_cast<const half8 *>(sc + 512 + qg * 128 + (b + 1) * 16);
+                        products(b + 1);
                     }
                 }
-                const half8 va0 = widen8<false>(vw[0], vw[1]);
-                const half8 va1 = widen8<false>(vw[2], vw[3]);
+                if (b + 2 < kBlocks) {
+                    load_v(b + 2);
+                }
 #pragma unroll
-                for (int rt = 0; rt < NTW; ++rt) {
-                    if (!KV8 || (b & 1) == 0) {
-                        scale_hilo_pk(ph[rt], pl[rt], vs, phs[rt], pls[rt]);
+                for (int m = 0; m < 2; ++m) {
+#pragma unroll
+                    for (int rt = 0; rt < NTW; ++rt) {
+                        acc[rt][b][m] = mfma16(va[b & 1][m], hi[set_of(b)][rt], acc[rt][b][m]);
                     }
-                    const half8 hi = phs[rt], lo = pls[rt];
-                    acc[rt][b][0] = mfma16(va0, hi, acc[rt][b][0]);
-                    acc[rt][b][1] = mfma16(va1, hi, acc[rt][b][1]);
-                    acc[rt][b][0] = mfma16(va0, lo, acc[rt][b][0]);
-                    acc[rt][b][1] = mfma16(va1, lo, acc[rt][b][1]);
+#pragma unroll
+                    for (int rt = 0; rt < NTW; ++rt) {
+                        acc[rt][b][m] = mfma16(va[b & 1][m], lo[set_of(b)][rt], acc[rt][b][m]);
+                    }
                 }
-                __builtin_amdgcn_sched_barrier(0); // one block's operands live at a time
+                if (b + 1 < kBlocks) { // four VALU instructions behind each MFMA
+#pragma unroll
+                    for (int m = 0; m < 4 * NTW; ++m) {
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
             issue_half(i + 1, 1);
             FNKV_PHASE(5);
