@@ -187,14 +187,13 @@ struct dec_plan {
     bool fold = false; // the stream kernel folds the splits itself (no merge launch)
 };
 
-dec_plan plan_decode(const kv_pool & p, int32_t n_seq, const int64_t * ctx, int32_t R) {
+dec_plan plan_decode(const kv_pool & p, int32_t n_seq, const int64_t * ctx, int32_t R, bool fine = true) {
     dec_plan pl;
     const int32_t cus = device_cus(p.device());
-    pl.split_tokens =
-        choose_split_stream(n_seq, ctx, p.h_kv(), cus, (R + 15) / 16);
-    // tuning knob for measurement: FNKV_SPLIT_TOKENS (a multiple of 32 from 256 to 2,048), read once per process
+    pl.split_tokens = choose_split_stream(n_seq, ctx, p.h_kv(), cus, (R + 15) / 16, fine);
+    // tuning knob for measurement: FNKV_SPLIT_TOKENS (a multiple of 32 from 256 to 4,096), read once per process
     static const int32_t split_knob = env_int_once("FNKV_SPLIT_TOKENS", 0);
-    if (split_knob >= kPageTokens && split_knob <= 8 * kPageTokens && split_knob % kTileTokens == 0) {
+    if (split_knob >= kPageTokens && split_knob <= kMaxSplitPages * kPageTokens && split_knob % kTileTokens == 0) {
         pl.split_tokens = split_knob;
     }
     pl.split0[0] = 0;
@@ -352,7 +351,11 @@ int decode_launch(const fnkv_pool * pool, int32_t n_seq, const int32_t * slots, 
             }
         }
     }
-    const dec_plan pl = plan_decode(*p, n_seq, ctx, R);
+    dec_plan pl = plan_decode(*p, n_seq, ctx, R);
+    if (ws_bytes < pl.fold_bytes + pl.po_bytes + pl.pml_bytes) {
+        // (a workspace sized for longer contexts can be smaller than the fine splits of short ones need)
+        pl = plan_decode(*p, n_seq, ctx, R, false);
+    }
     if (ws_bytes < pl.fold_bytes + pl.po_bytes + pl.pml_bytes) {
         set_error(name + ": workspace too small");
         return FNKV_ERR_ARG;

@@ -123,11 +123,12 @@ __device__ __forceinline__ int32_t page_of(const int32_t * table, bool active, i
     return table[active ? idx : 0];
 }
 
-// The tiles a dense workgroup walks, at most 64 (splits of at most 2,048 cells): lane i holds the physical page of walk
-// tile i, so a tile's page is a lane read.
+// The tiles a dense workgroup walks, at most 128 (splits of at most kMaxSplitPages pages): lane i holds the physical
+// pages of walk tiles i and 64 + i, so a tile's page is a lane read.
+constexpr int32_t kMaxSplitPages = 16;
 struct split_src {
     int32_t n_tiles = 0;
-    int32_t page_lane = 0;
+    int32_t page_lane = 0, page_hi = 0;
     int32_t g0 = 0, stride = 1; // walk tile i is the sequence's tile g0 + stride i
 
     // The split's own cells b .. e, or (strided) split j of the sequence's n takes its tiles j, j + n, ...; the strided
@@ -140,6 +141,7 @@ struct split_src {
             const int32_t tiles_cap = static_cast<int32_t>((a.ctx[s] + kTileTokens - 1) / kTileTokens);
             const int32_t cap_n = tiles_cap > j ? (tiles_cap - j + n - 1) / n : 0;
             page_lane = page_of(table, lane < cap_n, (j + n * lane) >> 3);
+            page_hi = page_of(table, 64 + lane < cap_n, (j + n * (64 + lane)) >> 3);
             g0 = j;
             stride = n;
             recount(ctx);
@@ -147,7 +149,8 @@ struct split_src {
             g0 = static_cast<int32_t>(b / kTileTokens);
             stride = 1;
             n_tiles = static_cast<int32_t>((e - b + kTileTokens - 1) / kTileTokens);
-            page_lane = page_of(table, lane < n_tiles, (g0 + stride * lane) >> 3);
+            page_lane = page_of(table, lane < n_tiles, (g0 + lane) >> 3);
+            page_hi = page_of(table, 64 + lane < n_tiles, (g0 + 64 + lane) >> 3);
         }
     }
     // A strided walk sized by the host's bound: its tile count for the sequence's actual context (read from the
@@ -161,15 +164,20 @@ struct split_src {
     // writes no output for its sequence (its partials carry a NaN max: the merge writes nothing for such a row).
     // Lanes past the walk take page 0 too. Every dense walk calls this once its tile count is final.
     __device__ __forceinline__ bool guard_unmapped(int32_t lane) {
-        const bool neg = lane < n_tiles && page_lane < 0;
+        const bool neg = lane < n_tiles && page_lane < 0, neg_hi = 64 + lane < n_tiles && page_hi < 0;
         if (neg || lane >= n_tiles) {
             page_lane = 0;
         }
-        return __any(neg);
+        if (neg_hi || 64 + lane >= n_tiles) {
+            page_hi = 0;
+        }
+        return __any(neg || neg_hi);
     }
     // byte offset of walk tile ti within the (layer, head) plane of the pool
     __device__ __forceinline__ int64_t tile_off(const pool_view & pv, int32_t ti) const {
-        const int32_t phys = __builtin_amdgcn_readlane(page_lane, ti);
+        const int32_t lo = __builtin_amdgcn_readlane(page_lane, ti & 63);
+        const int32_t hi = __builtin_amdgcn_readlane(page_hi, ti & 63);
+        const int32_t phys = ti < 64 ? lo : hi;
         return int64_t(phys) * pv.page_stride + int64_t((g0 + stride * ti) & 7) * kTileBytes;
     }
     // the first cell of walk tile ti
@@ -250,8 +258,9 @@ struct fused_prep; // gather.h
 void launch_merge(const merge_args & m, hipStream_t st);
 // host: the dense launch's one-stream-a-wave kernel for NT = 1 .. 3 row tiles (stream.hip)
 void launch_stream(int32_t device, int32_t NT, dim3 grid, const dec_args & a, hipStream_t st);
-// the split size (cells) of a dense launch run by the stream kernel with NT row tiles
-int32_t choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_kv, int32_t cus, int32_t NT);
+// the split size (cells) of a dense launch run by the stream kernel with NT row tiles; fine: kFineSplit is allowed
+constexpr int32_t kFineSplit = 128;
+int32_t choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_kv, int32_t cus, int32_t NT, bool fine);
 // a launch's depth read from device memory (the reference's depth word, attend.h:108): depth + T <= max_cells or
 // the launch writes nothing and ORs FNKV_DEV_ERR_DEPTH into *err
 struct dev_depth {

@@ -56,30 +56,34 @@ template <int NT> struct stream_shape {
     static constexpr int AUX = NT == 3 ? 0 : kStreamAux;
     static constexpr int SLOT = kTileBytes;          // a tile, in its HBM layout
     static constexpr int RING = WAVES * SLOT;        // 139,264 B
-    static constexpr int QOPS = NT * kBlocks * 1024; // the Q operands: [row tile][block][lane] 16 B
+    // the Q operands of row tiles 0 and 1, [row tile][block][lane] 16 B, and their per-block sums (the bias term's
+    // operand), [row tile][lane] 16 B; row tile 2's are in its waves' registers
+    static constexpr int QTILES = NT < 2 ? NT : 2;
+    static constexpr int QOPS = QTILES * kBlocks * 1024;
+    static constexpr int SIGS = QTILES * 1024;
     static constexpr int OSTRIDE = kHeadDim + 4;     // floats a row of the fold buffer
-    static constexpr int LDS = RING + QOPS; // the 8-wave fold reuses the tile slots
+    static constexpr int LDS = RING + QOPS + SIGS; // the 8-wave fold reuses the tile slots
     static_assert(LDS <= 160 * 1024, "LDS");
     // a half tile is 9 loads: 8 chunks of codes and half of the scales chunk; the wave waits for one half with the
     // other half's 9 issued after it
     static constexpr int HALF_LOADS = 9;
 };
 
-// S^T = K Q^T of one tile for NT row tiles from the K codes (kb) and the scales chunk (sc) in LDS: s_out[rt][h][r]
+// S^T = K Q^T of one tile for NT row tiles from the K codes (kb) and the scales chunk (sc) in LDS, the Q operands qo_at(rt, block) and the rows' per-block q sums
+// sig_at(rt): s_out[rt][h][r]
 // is the score (q . k, unscaled) of token 16 h + 4 qg + r against row 16 rt + j. Each block of K codes is widened once
 // and feeds the MFMAs of every row tile. The blocks run as a pipeline: beside block n + 1's MFMAs stand block n's scale
 // FMAs (one a score), block n + 2's widening and the LDS reads of the operands after those, interleaved with the MFMAs
 // (a wave that waits for a busy matrix core cannot reach VALU work that stands behind it). KV8: a chunk's two blocks are
 // one 64-value group with one scale, so their two MFMAs chain and the group takes one FMA a score.
-template <int NT, bool KV8>
-__device__ __forceinline__ void stream_scores(const uint8_t * kb, const uint8_t * sc, const uint8_t * qs,
-                                              const half8 (&sig)[NT], int32_t j, int32_t qg, int32_t lane,
+template <int NT, bool KV8, typename QOP, typename SIG>
+__device__ __forceinline__ void stream_scores(const uint8_t * kb, const uint8_t * sc, const QOP & qo_at,
+                                              const SIG & sig_at, int32_t j, int32_t qg, int32_t lane,
                                               floatx4 (&s_out)[NT][2]) {
     const half8 zero8 = {};
     const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
     // block n of the tile's 16 (half n / 8, block n % 8): its codes are words 2 (n & 1), + 1 of chunk n / 2
     auto kw_at = [&](int c) { return *reinterpret_cast<const u32x4 *>(kb + (c >> 2) * 4096 + (c & 3) * 1024 + lane * 16); };
-    auto qo_at = [&](int rt, int b) { return *reinterpret_cast<const half8 *>(qs + (rt * kBlocks + b) * 1024 + lane * 16); };
     u32x4 kw = kw_at(0);
     half8 ka[2], qo[NT];
     floatx4 t[2][NT];
@@ -117,7 +121,7 @@ __device__ __forceinline__ void stream_scores(const uint8_t * kb, const uint8_t 
             const half8 srow = qg < 2 ? *reinterpret_cast<const half8 *>(sc + (16 * h + j) * 16) : zero8;
 #pragma unroll
             for (int rt = 0; rt < NT; ++rt) {
-                acc_s[rt] = mfma16(srow, sig[rt], zero4) * -1152.0f;
+                acc_s[rt] = mfma16(srow, sig_at(rt), zero4) * -1152.0f;
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -455,19 +459,21 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
 
     // The Q operands of every row tile go into LDS once (the workgroup's waves share them: wave w loads operands w,
     // w + 8, ...); their loads are issued first, beside the page-table read
-    uint8_t * const qs = smem + SH::RING;
-    constexpr int PER = NT * kBlocks / WAVES;
+    uint8_t * const qs = smem + SH::RING, * const sigs = qs + SH::QOPS;
+    constexpr int PER = SH::QTILES * kBlocks / WAVES;
+    auto load_op = [&](int rt, int b) {
+        const int32_t row = rt * 16 + j < a.R ? rt * 16 + j : a.R - 1;
+        const int32_t t_row = row / a.G;
+        return *reinterpret_cast<const u32x4 *>(
+            a.q + ((int64_t(s) * a.T + t_row) * a.hq + int64_t(kvh) * a.G + row % a.G) * kHeadDim + b * kQK + 8 * qg);
+    };
     // (a padding row takes the last real row's q, loaded unconditionally: a load under a branch would make the
     // compiler wait for it before the page-table read; padding rows are computed like the others and never folded or
     // written)
     u32x4 qv[PER];
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-        const int32_t c = wave + e * WAVES, rt = c / kBlocks, b = c % kBlocks;
-        const int32_t row = rt * 16 + j < a.R ? rt * 16 + j : a.R - 1;
-        const int32_t t_row = row / a.G;
-        qv[e] = *reinterpret_cast<const u32x4 *>(
-            a.q + ((int64_t(s) * a.T + t_row) * a.hq + int64_t(kvh) * a.G + row % a.G) * kHeadDim + b * kQK + 8 * qg);
+        qv[e] = load_op((wave + e * WAVES) / kBlocks, (wave + e * WAVES) % kBlocks);
     }
     split_src src;
     src.init(a, table, split, begin, ctx < begin + a.split_tokens ? ctx : begin + a.split_tokens, lane, ctx);
@@ -548,18 +554,42 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
     // The walk and the fold for a wave holding row tiles RTB .. RTB + NTW - 1 (every wave passes the same barriers)
     auto run = [&](auto ntw_c, auto rtb_c) {
         constexpr int32_t NTW = decltype(ntw_c)::value, RTB = decltype(rtb_c)::value;
-        const uint8_t * const qw = qs + RTB * kBlocks * 1024; // this wave's row tiles' Q operands
+        // this wave's row tiles' Q operands and sums: in LDS, row tile 2's in registers
+        constexpr bool OWN = RTB == 2;
+        half8 q_own[OWN ? kBlocks : 1] = {}, sig_own = {};
+        if constexpr (OWN) {
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                q_own[b] = __builtin_bit_cast(half8, load_op(RTB, b));
+            }
+        }
+        auto qo_at = [&](int rt, int b) {
+            if constexpr (OWN) {
+                return q_own[b];
+            } else {
+                return *reinterpret_cast<const half8 *>(qs + (rt * kBlocks + b) * 1024 + lane * 16);
+            }
+        };
+        auto sig_at = [&](int rt) {
+            if constexpr (OWN) {
+                return sig_own;
+            } else {
+                return *reinterpret_cast<const half8 *>(sigs + rt * 1024 + lane * 16);
+            }
+        };
         // each lane's bias operands (the rows' per-block q sums) and each row's last visible cell
-        half8 sig[NTW];
         int64_t lim[NTW];
 #pragma unroll
         for (int rt = 0; rt < NTW; ++rt) {
             half8 qop[kBlocks];
 #pragma unroll
             for (int b = 0; b < kBlocks; ++b) {
-                qop[b] = *reinterpret_cast<const half8 *>(qw + (rt * kBlocks + b) * 1024 + lane * 16);
+                qop[b] = qo_at(rt, b);
             }
-            sig[rt] = q_sums(qop, qg);
+            sig_own = q_sums(qop, qg);
+            if constexpr (!OWN) { // (each wave that reads it writes it: the same values)
+                *reinterpret_cast<half8 *>(sigs + rt * 1024 + lane * 16) = sig_own;
+            }
             lim[rt] = ctx - a.T + t_of_row(a, RTB + rt, j);
         }
         floatx4 acc[NTW][kBlocks][2];
@@ -593,7 +623,7 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
             const uint8_t * kb = slot;
             const uint8_t * sc = kb + kKScales;
             floatx4 scv[NTW][2];
-            stream_scores<NTW, KV8>(kb, sc, qw, sig, j, qg, lane, scv);
+            stream_scores<NTW, KV8>(kb, sc, qo_at, sig_at, j, qg, lane, scv);
             issue_half(i + 1, 0); // the scores' reads of K(i) are done (their values are in registers)
             FNKV_PHASE(2);
             const int64_t tok0 = src.tok0(st + i * STREAMS);
@@ -834,25 +864,43 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
     FNKV_STAMP(4);
 }
 
-// The split size (cells) for these contexts: the fewest rounds of one workgroup a CU times a workgroup's time, which
-// is its waves' longest walk (the split's tiles over its tile streams, rounded up) plus a fixed cost (the ramp, the fold of the
-// waves and the partial's write, counted as three tiles); larger splits (fewer partials) win ties.
-int32_t choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_kv, int32_t cus, int32_t NT) {
+// The split size (cells) for these contexts. `fine` and splits of kFineSplit cells at most one a CU: those, so that each
+// of a workgroup's SIMDs holds one tile. A tile's products take a wave 1.1 us alone on its SIMD and 2.2 us beside
+// another's, and launches this small have CUs to spare: 16 heads on 2 KV heads, 4,096 cells 14.6 -> 12.9 us a launch
+// (merge included) at T = 1, 19.7 -> 16.8 at 3, 22.8 -> 20.2 at 5; 700 cells 13.3 -> 12.0; splits of 64 cells 13.3 at
+// 4,096, of 160 to 224 (two tiles on some SIMDs) 14.0 and more; at two rounds (16,384 cells) 128 cells lose, 19.5
+// against 15.5. Else the fewest rounds of one workgroup a CU times a workgroup's time, which is its waves' longest
+// walk (the split's tiles over its tile streams, rounded up) plus a fixed cost (the ramp, the fold of the waves and the
+// partial's write, counted as three tiles); larger splits (fewer partials) win ties. The longest split is what its
+// waves' page registers hold: a bound just past a round's 2,048-cell splits (262,401 cells) would otherwise take a
+// second round of half-size splits, 83.0 against 93.5 us a layer at T = 5.
+int32_t choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_kv, int32_t cus, int32_t NT, bool fine) {
+    int64_t tiles[FNKV_MAX_SEQS];
+    for (int32_t i = 0; i < n_seq; ++i) {
+        tiles[i] = (ctx[i] + kTileTokens - 1) / kTileTokens;
+    }
+    auto workgroups = [&](uint32_t split) { // of `split` tiles a split
+        int64_t n = 0;
+        for (int32_t i = 0; i < n_seq; ++i) {
+            // (32-bit divisions: these are most of what a plan costs the host)
+            n += tiles[i] <= INT32_MAX ? (static_cast<uint32_t>(tiles[i]) + split - 1) / split
+                                       : (tiles[i] + split - 1) / split;
+        }
+        return n * h_kv;
+    };
+    if (fine && workgroups(kFineSplit / kTileTokens) <= cus) {
+        return kFineSplit;
+    }
+    // sizes between two multiples of the streams' tiles cost what the upper one does and take more workgroups
     const int32_t streams = NT == 3 ? stream_shape<3>::STREAMS : stream_shape<1>::STREAMS;
     int32_t best = kPageTokens;
     int64_t best_cost = INT64_MAX;
-    for (int32_t sz = kPageTokens; sz <= 8 * kPageTokens; sz += kTileTokens) {
-        int64_t wgs = 0;
-        for (int32_t i = 0; i < n_seq; ++i) {
-            wgs += (ctx[i] + sz - 1) / sz;
-        }
-        wgs *= h_kv;
-        const int64_t rounds = (wgs + cus - 1) / cus;
-        const int64_t wave_tiles = (sz / kTileTokens + streams - 1) / streams;
-        const int64_t cost = rounds * (wave_tiles + 3);
+    for (int32_t t = kPageTokens / kTileTokens; t <= kMaxSplitPages * kPageTokens / kTileTokens; t += streams) {
+        const int64_t rounds = (workgroups(static_cast<uint32_t>(t)) + cus - 1) / cus;
+        const int64_t cost = rounds * (t / streams + 3);
         if (cost <= best_cost) {
             best_cost = cost;
-            best = sz;
+            best = t * kTileTokens;
         }
     }
     return best;
