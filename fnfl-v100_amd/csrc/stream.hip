@@ -24,6 +24,9 @@
 //     the LDS reads of the one after ahead of it) and the row tiles' softmax chains side by side: 16 heads on 2 KV
 //     heads, 4,096 cells 14.7 -> 14.3 us a layer, 262,144 cells at 5 rows 93.5 -> 92.0, four sequences of 8K to 64K at
 //     3 rows 37.8 -> 37.5 (the loads bound those: without any of the products a layer still takes 32 us);
+//   * what a short walk would wait for besides its tiles is left out (4,096 cells 13.1 -> 12.4 us a layer, 262,144 cells
+//     51.7 -> 50.8): loads past the walk's end, a wave without tiles, the fold of the streams that held none, block by
+//     block LDS reads where one row tile leaves the registers to read a half at once;
 //   * one MFMA pair a tile against the V scales (and a row of ones) gives each row's V bias sums and its l;
 //   * a KV8 pool (group-64 scales, stored at both blocks of a group) takes the KV8 instantiation: a group's two score
 //     MFMAs chain before its one scale FMA, and its P x V-scale products serve both of its blocks;
@@ -60,7 +63,7 @@ template <int NT> struct stream_shape {
     // operand), [row tile][lane] 16 B; row tile 2's are in its waves' registers
     static constexpr int QTILES = NT < 2 ? NT : 2;
     static constexpr int QOPS = QTILES * kBlocks * 1024;
-    static constexpr int SIGS = QTILES * 1024;
+    static constexpr int SIGS = NT == 1 ? 0 : QTILES * 1024;
     static constexpr int OSTRIDE = kHeadDim + 4;     // floats a row of the fold buffer
     static constexpr int LDS = RING + QOPS + SIGS; // the 8-wave fold reuses the tile slots
     static_assert(LDS <= 160 * 1024, "LDS");
@@ -84,12 +87,33 @@ __device__ __forceinline__ void stream_scores(const uint8_t * kb, const uint8_t 
     const floatx4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
     // block n of the tile's 16 (half n / 8, block n % 8): its codes are words 2 (n & 1), + 1 of chunk n / 2
     auto kw_at = [&](int c) { return *reinterpret_cast<const u32x4 *>(kb + (c >> 2) * 4096 + (c & 3) * 1024 + lane * 16); };
-    u32x4 kw = kw_at(0);
+    // one row tile has the registers to read all of the tile's K half at once: block by block, an LDS read's latency
+    // (about 120 cycles) is all that a block's step takes where the SIMD has no other wave to run
+    constexpr bool ALL = NT == 1;
+    u32x4 kw[ALL ? 8 : 1];
     half8 ka[2], qo[NT];
     floatx4 t[2][NT];
-    half8 ks[4];
+    half8 ks[ALL ? 2 : 1][4], srow[ALL ? 2 : 1];
     floatx4 acc_s[NT];
-    auto widen = [&](int n) { ka[n & 1] = widen8<false>(kw[2 * (n & 1)], kw[2 * (n & 1) + 1]); };
+    auto widen = [&](int n) {
+        const u32x4 & w = kw[ALL ? n >> 1 : 0];
+        ka[n & 1] = widen8<false>(w[2 * (n & 1)], w[2 * (n & 1) + 1]);
+    };
+    auto load_scales = [&](int h) { // a half's token scales; A of the bias MFMA: the token row's scales (lanes qg < 2)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            ks[ALL ? h : 0][r] = *reinterpret_cast<const half8 *>(sc + (16 * h + 4 * qg + r) * 16);
+        }
+        srow[ALL ? h : 0] = qg < 2 ? *reinterpret_cast<const half8 *>(sc + (16 * h + j) * 16) : zero8;
+    };
+#pragma unroll
+    for (int c = 0; c < (ALL ? 8 : 1); ++c) {
+        kw[c] = kw_at(c);
+    }
+    if constexpr (ALL) {
+        load_scales(0);
+        load_scales(1);
+    }
     auto load_q = [&](int n) {
 #pragma unroll
         for (int rt = 0; rt < NT; ++rt) {
@@ -106,22 +130,22 @@ __device__ __forceinline__ void stream_scores(const uint8_t * kb, const uint8_t 
     widen(0);
     widen(1);
     load_q(0);
-    kw = kw_at(1);
+    if constexpr (!ALL) {
+        kw[0] = kw_at(1);
+    }
     products(0);
     load_q(1);
 #pragma unroll
     for (int n = 0; n < 16; ++n) {
         const int h = n >> 3, b = n & 7;
         if (b == 0) { // a half starts: its scales, and the bias term (-1152 times it) that its scores start from
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                ks[r] = *reinterpret_cast<const half8 *>(sc + (16 * h + 4 * qg + r) * 16);
+            if constexpr (!ALL) {
+                load_scales(h);
             }
-            // A = the token row's K scales (lanes qg < 2), B = the row's per-block q sums (hi, lo)
-            const half8 srow = qg < 2 ? *reinterpret_cast<const half8 *>(sc + (16 * h + j) * 16) : zero8;
+            // B = the row's per-block q sums (hi, lo)
 #pragma unroll
             for (int rt = 0; rt < NT; ++rt) {
-                acc_s[rt] = mfma16(srow, sig_at(rt), zero4) * -1152.0f;
+                acc_s[rt] = mfma16(srow[ALL ? h : 0], sig_at(rt), zero4) * -1152.0f;
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -132,8 +156,8 @@ __device__ __forceinline__ void stream_scores(const uint8_t * kb, const uint8_t 
             widen(n + 2);
             load_q(n + 2);
         }
-        if ((n & 1) == 1 && n + 3 < 16) {
-            kw = kw_at((n + 3) >> 1);
+        if (!ALL && (n & 1) == 1 && n + 3 < 16) {
+            kw[0] = kw_at((n + 3) >> 1);
         }
         if (!KV8 || (n & 1) == 1) {
             const int o = KV8 ? (n >> 1) & 1 : n & 1;
@@ -141,7 +165,7 @@ __device__ __forceinline__ void stream_scores(const uint8_t * kb, const uint8_t 
             for (int rt = 0; rt < NT; ++rt) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    acc_s[rt][r] = __builtin_fmaf(static_cast<float>(ks[r][b]), t[o][rt][r], acc_s[rt][r]);
+                    acc_s[rt][r] = __builtin_fmaf(static_cast<float>(ks[ALL ? h : 0][r][b]), t[o][rt][r], acc_s[rt][r]);
                 }
                 __asm__ volatile("" : "+v"(acc_s[rt])); // pin the FMAs here: two blocks' products live at a time
             }
@@ -513,23 +537,19 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
     const uint8_t * layer_base = pv.base + int64_t(a.layer) * pv.layer_stride + int64_t(kvh) * kPageBlock;
     uint8_t * const slot = smem + wave * SH::SLOT;
     const int32_t lane16 = lane * 16;
-    // iteration i's tile; past the wave's last tile a placeholder (the first tile, every lane reading its first
-    // 16 bytes of each chunk), so every iteration issues the same loads and the waits are fixed counts
-    auto tile_at = [&](int32_t i) -> const uint8_t * {
-        const int32_t ti = i < n_w ? st + i * STREAMS : 0;
-        return layer_base + src.tile_off(pv, n_tiles > 0 ? ti : 0);
+    auto tile_at = [&](int32_t i) -> const uint8_t * { // iteration i's tile
+        return layer_base + src.tile_off(pv, st + i * STREAMS);
     };
     // half V = 0: the K codes (chunks 0-7) and the K scales (the scales chunk's lanes 0-31); V = 1: the V codes
     // (chunks 8-15) and the V scales (its lanes 32-63)
     auto issue_half = [&](int32_t i, int32_t V) {
         const rsrc_t r = make_rsrc(tile_at(i), kTileBytes);
-        const int32_t voff = i < n_w ? lane16 : 0;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            buf_lds16<SH::AUX>(r, slot + (8 * V + c) * 1024, voff, (8 * V + c) * 1024);
+            buf_lds16<SH::AUX>(r, slot + (8 * V + c) * 1024, lane16, (8 * V + c) * 1024);
         }
         if ((lane >> 5) == V) {
-            buf_lds16<SH::AUX>(r, slot + kKScales, voff, kKScales);
+            buf_lds16<SH::AUX>(r, slot + kKScales, lane16, kKScales);
         }
         keep_issued();
     };
@@ -554,197 +574,217 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
     // The walk and the fold for a wave holding row tiles RTB .. RTB + NTW - 1 (every wave passes the same barriers)
     auto run = [&](auto ntw_c, auto rtb_c) {
         constexpr int32_t NTW = decltype(ntw_c)::value, RTB = decltype(rtb_c)::value;
-        // this wave's row tiles' Q operands and sums: in LDS, row tile 2's in registers
-        constexpr bool OWN = RTB == 2;
-        half8 q_own[OWN ? kBlocks : 1] = {}, sig_own = {};
-        if constexpr (OWN) {
-#pragma unroll
-            for (int b = 0; b < kBlocks; ++b) {
-                q_own[b] = __builtin_bit_cast(half8, load_op(RTB, b));
-            }
-        }
-        auto qo_at = [&](int rt, int b) {
-            if constexpr (OWN) {
-                return q_own[b];
-            } else {
-                return *reinterpret_cast<const half8 *>(qs + (rt * kBlocks + b) * 1024 + lane * 16);
-            }
-        };
-        auto sig_at = [&](int rt) {
-            if constexpr (OWN) {
-                return sig_own;
-            } else {
-                return *reinterpret_cast<const half8 *>(sigs + rt * 1024 + lane * 16);
-            }
-        };
-        // each lane's bias operands (the rows' per-block q sums) and each row's last visible cell
-        int64_t lim[NTW];
-#pragma unroll
-        for (int rt = 0; rt < NTW; ++rt) {
-            half8 qop[kBlocks];
-#pragma unroll
-            for (int b = 0; b < kBlocks; ++b) {
-                qop[b] = qo_at(rt, b);
-            }
-            sig_own = q_sums(qop, qg);
-            if constexpr (!OWN) { // (each wave that reads it writes it: the same values)
-                *reinterpret_cast<half8 *>(sigs + rt * 1024 + lane * 16) = sig_own;
-            }
-            lim[rt] = ctx - a.T + t_of_row(a, RTB + rt, j);
-        }
         floatx4 acc[NTW][kBlocks][2];
-        floatx4 lv[NTW]; // lane (row j, qg): rows 4 qg + e of sum_t P s_v[t][b] (b < 8) and sum_t P (row 8)
-        float m_run[NTW];
+        float m_run[NTW], l_row[NTW];
+        if (n_w > 0) { // (a wave without tiles leaves its SIMD to the others)
+            // this wave's row tiles' Q operands and sums: in LDS, a wave's only row tile's in registers
+            constexpr bool OWN = NTW == 1;
+            half8 q_own[OWN ? kBlocks : 1] = {}, sig_own = {};
+            if constexpr (OWN) {
 #pragma unroll
-        for (int rt = 0; rt < NTW; ++rt) {
-            lv[rt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-            m_run[rt] = kNegInf;
-#pragma unroll
-            for (int b = 0; b < kBlocks; ++b) {
-                acc[rt][b][0] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-                acc[rt][b][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int b = 0; b < kBlocks; ++b) {
+                    if constexpr (RTB == 2) {
+                        q_own[b] = __builtin_bit_cast(half8, load_op(RTB, b));
+                    } else {
+                        q_own[b] = *reinterpret_cast<const half8 *>(qs + b * 1024 + lane * 16);
+                    }
+                }
             }
-        }
+            auto qo_at = [&](int rt, int b) {
+                if constexpr (OWN) {
+                    return q_own[b];
+                } else {
+                    return *reinterpret_cast<const half8 *>(qs + (rt * kBlocks + b) * 1024 + lane * 16);
+                }
+            };
+            auto sig_at = [&](int rt) {
+                if constexpr (OWN) {
+                    return sig_own;
+                } else {
+                    return *reinterpret_cast<const half8 *>(sigs + rt * 1024 + lane * 16);
+                }
+            };
+            // each lane's bias operands (the rows' per-block q sums) and each row's last visible cell
+            int64_t lim[NTW];
+#pragma unroll
+            for (int rt = 0; rt < NTW; ++rt) {
+                half8 qop[kBlocks];
+#pragma unroll
+                for (int b = 0; b < kBlocks; ++b) {
+                    qop[b] = qo_at(rt, b);
+                }
+                sig_own = q_sums(qop, qg);
+                if constexpr (!OWN) { // (each wave that reads it writes it: the same values)
+                    *reinterpret_cast<half8 *>(sigs + rt * 1024 + lane * 16) = sig_own;
+                }
+                lim[rt] = ctx - a.T + t_of_row(a, RTB + rt, j);
+            }
+            floatx4 lv[NTW]; // lane (row j, qg): rows 4 qg + e of sum_t P s_v[t][b] (b < 8) and sum_t P (row 8)
+#pragma unroll
+            for (int rt = 0; rt < NTW; ++rt) {
+                lv[rt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                m_run[rt] = kNegInf;
+#pragma unroll
+                for (int b = 0; b < kBlocks; ++b) {
+                    acc[rt][b][0] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                    acc[rt][b][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+            }
 
-        // Iteration i: wait for K(i), scores, issue K(i + 1), softmax, wait for V(i), PV, issue V(i + 1). V(0) is
-        // issued once K(0) has landed, so it loads under tile 0's scores.
-        if (n_w > 0) {
+            // Iteration i: wait for K(i), scores, issue K(i + 1), softmax, wait for V(i), PV, issue V(i + 1). V(0) is
+            // issued once K(0) has landed, so it loads under tile 0's scores.
             wait_vmcnt<0>();
             issue_half(0, 1);
-        }
-        FNKV_PHASE_DECL();
-        for (int32_t i = 0; i < n_w; ++i) {
-            FNKV_PHASE(0 + (i > 0 ? 7 : 0));
-            wait_vmcnt<SH::HALF_LOADS>(); // K(i) has landed (V(i) may be pending)
-            FNKV_PHASE(1);
-            // the scores and the softmax are the longer dependent chain: their wave issues first on a shared SIMD,
-            // so the two waves of a SIMD alternate phases rather than one running ahead
-            __builtin_amdgcn_s_setprio(1);
-            const uint8_t * kb = slot;
-            const uint8_t * sc = kb + kKScales;
-            floatx4 scv[NTW][2];
-            stream_scores<NTW, KV8>(kb, sc, qo_at, sig_at, j, qg, lane, scv);
-            issue_half(i + 1, 0); // the scores' reads of K(i) are done (their values are in registers)
-            FNKV_PHASE(2);
-            const int64_t tok0 = src.tok0(st + i * STREAMS);
-            half8 ph[NTW], pl[NTW];
-            {
-                int32_t lim_rel[NTW];
-                float alpha[NTW];
-                bool same = true;
-#pragma unroll
-                for (int rt = 0; rt < NTW; ++rt) {
-                    const int64_t lr = lim[rt] - tok0;
-                    lim_rel[rt] = lr > 64 ? 64 : static_cast<int32_t>(lr < -1 ? -1 : lr);
+            FNKV_PHASE_DECL();
+            for (int32_t i = 0; i < n_w; ++i) {
+                FNKV_PHASE(0 + (i > 0 ? 7 : 0));
+                wait_vmcnt<SH::HALF_LOADS>(); // K(i) has landed (V(i) may be pending)
+                FNKV_PHASE(1);
+                // the scores and the softmax are the longer dependent chain: their wave issues first on a shared SIMD,
+                // so the two waves of a SIMD alternate phases rather than one running ahead
+                __builtin_amdgcn_s_setprio(1);
+                const uint8_t * kb = slot;
+                const uint8_t * sc = kb + kKScales;
+                floatx4 scv[NTW][2];
+                stream_scores<NTW, KV8>(kb, sc, qo_at, sig_at, j, qg, lane, scv);
+                const bool more = i + 1 < n_w;
+                if (more) { // the scores' reads of K(i) are done (their values are in registers)
+                    issue_half(i + 1, 0);
                 }
-                stream_softmax<NTW>(scv, lim_rel, a.c2, qg, m_run, ph, pl, alpha);
-#pragma unroll
-                for (int rt = 0; rt < NTW; ++rt) {
-                    same = same && alpha[rt] == 1.0f;
-                }
-                if (!__all(same)) {
+                FNKV_PHASE(2);
+                const int64_t tok0 = src.tok0(st + i * STREAMS);
+                half8 ph[NTW], pl[NTW];
+                {
+                    int32_t lim_rel[NTW];
+                    float alpha[NTW];
+                    bool same = true;
 #pragma unroll
                     for (int rt = 0; rt < NTW; ++rt) {
+                        const int64_t lr = lim[rt] - tok0;
+                        lim_rel[rt] = lr > 64 ? 64 : static_cast<int32_t>(lr < -1 ? -1 : lr);
+                    }
+                    stream_softmax<NTW>(scv, lim_rel, a.c2, qg, m_run, ph, pl, alpha);
 #pragma unroll
-                        for (int b = 0; b < kBlocks; ++b) {
-                            acc[rt][b][0] *= alpha[rt];
-                            acc[rt][b][1] *= alpha[rt];
+                    for (int rt = 0; rt < NTW; ++rt) {
+                        same = same && alpha[rt] == 1.0f;
+                    }
+                    if (!__all(same)) {
+#pragma unroll
+                        for (int rt = 0; rt < NTW; ++rt) {
+#pragma unroll
+                            for (int b = 0; b < kBlocks; ++b) {
+                                acc[rt][b][0] *= alpha[rt];
+                                acc[rt][b][1] *= alpha[rt];
+                            }
+                            lv[rt] *= alpha[rt];
                         }
-                        lv[rt] *= alpha[rt];
                     }
                 }
-            }
-            FNKV_PHASE(3);
-            __builtin_amdgcn_s_setprio(0);
-            wait_vmcnt<SH::HALF_LOADS>(); // V(i) has landed (K(i + 1) may be pending)
-            FNKV_PHASE(4);
-            // PV as the scores' pipeline: beside block b's MFMAs stand block b + 1's widened codes and P x V-scale
-            // products, and the LDS reads of block b + 2. KV8: a group's two blocks share their scales and products.
-            u32x4 vw = *reinterpret_cast<const u32x4 *>(kb + kVCodes + lane * 16);
-            half8 vs = *reinterpret_cast<const half8 *>(sc + 512 + qg * 128);
-            half8 va[2][2], hi[2][NTW], lo[2][NTW]; // [parity]
-            auto widen_v = [&](int b) {
-                va[b & 1][0] = widen8<false>(vw[0], vw[1]);
-                va[b & 1][1] = widen8<false>(vw[2], vw[3]);
-            };
-            auto set_of = [](int b) { return KV8 ? (b >> 1) & 1 : b & 1; };
-            auto products = [&](int b) {
+                FNKV_PHASE(3);
+                __builtin_amdgcn_s_setprio(0);
+                if (more) { // V(i) has landed (K(i + 1) may be pending)
+                    wait_vmcnt<SH::HALF_LOADS>();
+                } else {
+                    wait_vmcnt<0>();
+                }
+                FNKV_PHASE(4);
+                // PV as the scores' pipeline: beside block b's MFMAs stand block b + 1's widened codes and P x V-scale
+                // products, and the LDS reads of block b + 2. KV8: a group's two blocks share their scales and products.
+                constexpr bool ALL = NTW == 1; // (the scores' reason)
+                u32x4 vw[ALL ? kBlocks : 1];
+                half8 vs[ALL ? kBlocks : 1];
+                half8 va[2][2], hi[2][NTW], lo[2][NTW]; // [parity]
+                auto widen_v = [&](int b) {
+                    const u32x4 & w = vw[ALL ? b : 0];
+                    va[b & 1][0] = widen8<false>(w[0], w[1]);
+                    va[b & 1][1] = widen8<false>(w[2], w[3]);
+                };
+                auto set_of = [](int b) { return KV8 ? (b >> 1) & 1 : b & 1; };
+                auto products = [&](int b) {
+#pragma unroll
+                    for (int rt = 0; rt < NTW; ++rt) {
+                        scale_hilo_pk(ph[rt], pl[rt], vs[ALL ? b : 0], hi[set_of(b)][rt], lo[set_of(b)][rt]);
+                    }
+                };
+                auto load_v = [&](int b) {
+                    vw[ALL ? b : 0] = *reinterpret_cast<const u32x4 *>(kb + kVCodes + b * 1024 + lane * 16);
+                    if (!KV8 || (b & 1) == 0) {
+                        vs[ALL ? b : 0] = *reinterpret_cast<const half8 *>(sc + 512 + qg * 128 + b * 16);
+                    }
+                };
+#pragma unroll
+                for (int b = 0; b < (ALL ? kBlocks : 1); ++b) {
+                    load_v(b);
+                }
+                // A of the bias MFMAs: lane (block j < 8, qg) holds s_v[token(qg, slot)][j], lanes j = 8 ones (l)
+                const half8 sva =
+                    j < 8 ? *reinterpret_cast<const half8 *>(sc + 512 + qg * 128 + j * 16) : j == 8 ? ones8 : zero8;
 #pragma unroll
                 for (int rt = 0; rt < NTW; ++rt) {
-                    scale_hilo_pk(ph[rt], pl[rt], vs, hi[set_of(b)][rt], lo[set_of(b)][rt]);
+                    lv[rt] = mfma16(sva, ph[rt], lv[rt]);
                 }
-            };
-            auto load_v = [&](int b) {
-                vw = *reinterpret_cast<const u32x4 *>(kb + kVCodes + b * 1024 + lane * 16);
-                if (!KV8 || (b & 1) == 0) {
-                    vs = *reinterpret_cast<const half8 *>(sc + 512 + qg * 128 + b * 16);
+                widen_v(0);
+                products(0);
+#pragma unroll
+                for (int rt = 0; rt < NTW; ++rt) {
+                    lv[rt] = mfma16(sva, pl[rt], lv[rt]);
                 }
-            };
-            // A of the bias MFMAs: lane (block j < 8, qg) holds s_v[token(qg, slot)][j], lanes j = 8 ones (l)
-            const half8 sva =
-                j < 8 ? *reinterpret_cast<const half8 *>(sc + 512 + qg * 128 + j * 16) : j == 8 ? ones8 : zero8;
-#pragma unroll
-            for (int rt = 0; rt < NTW; ++rt) {
-                lv[rt] = mfma16(sva, ph[rt], lv[rt]);
-            }
-            widen_v(0);
-            products(0);
-#pragma unroll
-            for (int rt = 0; rt < NTW; ++rt) {
-                lv[rt] = mfma16(sva, pl[rt], lv[rt]);
-            }
-            load_v(1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int b = 0; b < kBlocks; ++b) {
-                if (b + 1 < kBlocks) {
-                    widen_v(b + 1);
-                    if (!KV8 || (b & 1) == 1) {
-                        products(b + 1);
-                    }
-                }
-                if (b + 2 < kBlocks) {
-                    load_v(b + 2);
-                }
-#pragma unroll
-                for (int m = 0; m < 2; ++m) {
-#pragma unroll
-                    for (int rt = 0; rt < NTW; ++rt) {
-                        acc[rt][b][m] = mfma16(va[b & 1][m], hi[set_of(b)][rt], acc[rt][b][m]);
-                    }
-#pragma unroll
-                    for (int rt = 0; rt < NTW; ++rt) {
-                        acc[rt][b][m] = mfma16(va[b & 1][m], lo[set_of(b)][rt], acc[rt][b][m]);
-                    }
-                }
-                if (b + 1 < kBlocks) { // four VALU instructions behind each MFMA
-#pragma unroll
-                    for (int m = 0; m < 4 * NTW; ++m) {
-                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
-                    }
+                if constexpr (!ALL) {
+                    load_v(1);
                 }
                 __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int b = 0; b < kBlocks; ++b) {
+                    if (b + 1 < kBlocks) {
+                        widen_v(b + 1);
+                        if (!KV8 || (b & 1) == 1) {
+                            products(b + 1);
+                        }
+                    }
+                    if (!ALL && b + 2 < kBlocks) {
+                        load_v(b + 2);
+                    }
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) {
+#pragma unroll
+                        for (int rt = 0; rt < NTW; ++rt) {
+                            acc[rt][b][m] = mfma16(va[b & 1][m], hi[set_of(b)][rt], acc[rt][b][m]);
+                        }
+#pragma unroll
+                        for (int rt = 0; rt < NTW; ++rt) {
+                            acc[rt][b][m] = mfma16(va[b & 1][m], lo[set_of(b)][rt], acc[rt][b][m]);
+                        }
+                    }
+                    if (b + 1 < kBlocks) { // four VALU instructions behind each MFMA
+#pragma unroll
+                        for (int m = 0; m < 4 * NTW; ++m) {
+                            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (more) {
+                    issue_half(i + 1, 1);
+                }
+                FNKV_PHASE(5);
             }
-            issue_half(i + 1, 1);
-            FNKV_PHASE(5);
-        }
-        FNKV_PHASE_STORE();
-        wait_vmcnt<0>();
-        FNKV_STAMP_WAVE();
+            FNKV_PHASE_STORE();
+            wait_vmcnt<0>();
+            FNKV_STAMP_WAVE();
 
-        // the V bias: acc[rt][b] carries 1152 lv[rt][b]; lv[rt][b] of this lane's row sits in lane (j, b / 4),
-        // element b % 4; the row's l in lane (j, 2), element 0
-        float l_row[NTW];
+            // the V bias: acc[rt][b] carries 1152 lv[rt][b]; lv[rt][b] of this lane's row sits in lane (j, b / 4),
+            // element b % 4; the row's l in lane (j, 2), element 0
 #pragma unroll
-        for (int rt = 0; rt < NTW; ++rt) {
+            for (int rt = 0; rt < NTW; ++rt) {
 #pragma unroll
-            for (int b = 0; b < kBlocks; ++b) {
-                const float lb = __shfl(lv[rt][b & 3], j + 16 * (b >> 2));
-                acc[rt][b][0] -= 1152.0f * lb;
-                acc[rt][b][1] -= 1152.0f * lb;
+                for (int b = 0; b < kBlocks; ++b) {
+                    const float lb = __shfl(lv[rt][b & 3], j + 16 * (b >> 2));
+                    acc[rt][b][0] -= 1152.0f * lb;
+                    acc[rt][b][1] -= 1152.0f * lb;
+                }
+                l_row[rt] = __shfl(lv[rt][0], j + 32);
             }
-            l_row[rt] = __shfl(lv[rt][0], j + 32);
         }
 
         // ---- fold the STREAMS waves holding each row tile (fixed order), then the workgroup's row: the output itself
@@ -757,9 +797,20 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
         static_assert((ML + 16 * 2) * 4 <= SH::SLOT, "a row tile's fold buffer fits a tile slot");
         constexpr int32_t PASSES = SH::GROUPS == 1 ? NT : 2;
         float * const mine = reinterpret_cast<float *>(slot);
+        // the streams folded: all, or the first half where no other holds a tile (a wave without tiles among them
+        // writes what a walk that sees nothing would)
+        const int32_t n_fold = n_tiles > STREAMS / 2 ? STREAMS : STREAMS / 2;
 #pragma unroll
         for (int32_t k = 0; k < PASSES; ++k) {
-            if (k < NTW) {
+            if (k < NTW && st < n_fold) {
+                if (n_w == 0) {
+                    m_run[k] = kNegInf;
+                    l_row[k] = 0.0f;
+#pragma unroll
+                    for (int b = 0; b < kBlocks; ++b) {
+                        acc[k][b][0] = acc[k][b][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+                }
                 if ((RTB + k) * 16 + j < a.R) { // padding rows are not folded
 #pragma unroll
                     for (int b = 0; b < kBlocks; ++b) {
@@ -794,29 +845,36 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
                     continue;
                 }
                 const float * const hold = reinterpret_cast<const float *>(smem + g * STREAMS * SH::SLOT);
-                float2 mlw[STREAMS];
-                float Mr = kNegInf;
-#pragma unroll
-                for (int w = 0; w < STREAMS; ++w) {
-                    mlw[w] = *reinterpret_cast<const float2 *>(hold + w * (SH::SLOT / 4) + ML + 2 * rrow);
-                    Mr = fmaxf(Mr, mlw[w].x);
-                }
-                const float Mr_use = Mr == kNegInf ? 0.0f : Mr;
-                float L = 0.0f;
+                float Mr = kNegInf, L = 0.0f;
                 floatx4 sum[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+                auto fold = [&](auto n_c) {
+                    constexpr int32_t N = decltype(n_c)::value;
+                    float2 mlw[N];
 #pragma unroll
-                for (int w = 0; w < STREAMS; ++w) {
-                    const float f = __builtin_amdgcn_exp2f(mlw[w].x - Mr_use);
-                    L = __builtin_fmaf(mlw[w].y, f, L);
+                    for (int w = 0; w < N; ++w) {
+                        mlw[w] = *reinterpret_cast<const float2 *>(hold + w * (SH::SLOT / 4) + ML + 2 * rrow);
+                        Mr = fmaxf(Mr, mlw[w].x);
+                    }
+                    const float Mr_use = Mr == kNegInf ? 0.0f : Mr;
 #pragma unroll
-                    for (int c = 0; c < 2; ++c) {
-                        const floatx4 v =
-                            *reinterpret_cast<const floatx4 *>(hold + w * (SH::SLOT / 4) + rrow * OS + c0 + 128 * c);
+                    for (int w = 0; w < N; ++w) {
+                        const float f = __builtin_amdgcn_exp2f(mlw[w].x - Mr_use);
+                        L = __builtin_fmaf(mlw[w].y, f, L);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            sum[c][e] = __builtin_fmaf(v[e], f, sum[c][e]);
+                        for (int c = 0; c < 2; ++c) {
+                            const floatx4 v = *reinterpret_cast<const floatx4 *>(hold + w * (SH::SLOT / 4) +
+                                                                                 rrow * OS + c0 + 128 * c);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                sum[c][e] = __builtin_fmaf(v[e], f, sum[c][e]);
+                            }
                         }
                     }
+                };
+                if (n_fold == STREAMS) {
+                    fold(std::integral_constant<int32_t, STREAMS>());
+                } else {
+                    fold(std::integral_constant<int32_t, STREAMS / 2>());
                 }
                 if (unmapped) {
                     Mr = __builtin_nanf(""); // the merge (or the fold) writes nothing for this row
