@@ -194,7 +194,9 @@ __device__ __forceinline__ void issue_tile(const fnkv_datc_attend_args & a, cons
         const uint32_t off = c >= 0 ? static_cast<uint32_t>(c) * 512u + 16u * static_cast<uint32_t>(g) : kOob;
 #pragma unroll
         for (int32_t j = 0; j < 8; ++j) {
-            kt.r[h][j] = buf_load16(rk, static_cast<int32_t>(off), 64 * j);
+            // half a 128-byte line a cell: without the streaming bit, the next slice's load finds the other half in
+            // the vector L1 (196,600 cells: 45.2 -> 44.6 us a step; the V rows' whole lines stream, 46.8 without)
+            kt.r[h][j] = buf_load16<0>(rk, static_cast<int32_t>(off), 64 * j);
         }
     }
 #pragma unroll
@@ -502,16 +504,18 @@ __global__ __launch_bounds__(64 * kWaves, 1) void datc_attend_kernel(fnkv_datc_a
     }
     __syncthreads();
     float * part = reinterpret_cast<float *>(a.part) + static_cast<int64_t>(b) * kPartFloats;
+    // thread -> values 4 c .. + 3 of heads wave, wave + 4, wave + 8, the waves' rows summed in order
     const int32_t d = static_cast<int32_t>(threadIdx.x);
-    const float * of = reinterpret_cast<const float *>(smem);
+    const float * of = reinterpret_cast<const float *>(smem) + 4 * lane;
 #pragma unroll
-    for (int32_t hh = 0; hh < kHeads; ++hh) {
-        float acc = of[hh * kOStride + d];
+    for (int32_t i = 0; i < kHeads / kWaves; ++i) {
+        const int32_t hh = wave + kWaves * i;
+        floatx4 acc = *reinterpret_cast<const floatx4 *>(of + hh * kOStride);
 #pragma unroll
         for (int32_t w = 1; w < kWaves; ++w) {
-            acc += of[w * kHeads * kOStride + hh * kOStride + d];
+            acc += *reinterpret_cast<const floatx4 *>(of + w * kHeads * kOStride + hh * kOStride);
         }
-        part[hh * kD + d] = acc;
+        *reinterpret_cast<floatx4 *>(part + hh * kD + 4 * lane) = acc;
     }
     if (threadIdx.x < kHeads) {
         float Mh = -INFINITY;
@@ -530,6 +534,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void datc_attend_kernel(fnkv_datc_a
     DATC_STAMP(b, 3);
 }
 
+// (latency bound: its wave reductions and the run's on the VALU in place of LDS shuffles, and the workgroup's partial
+// written four values a lane, took a step at 4,096 cells from 14.0 to 13.3 us, one at 196,600 from 44.4 to 43.9)
 // the fold of (head h, values 32 r .. 32 r + 31): the active partials in workgroup order, the gate, the F32 output and
 // its activation-format run (act_run). Thread t takes partials t / 32 + 8 i of value t % 32 and issues all its loads
 // before the reductions that weigh them.
@@ -557,18 +563,14 @@ __global__ __launch_bounds__(256) void datc_fold_kernel(fnkv_datc_attend_args a,
     }
     const float m_raw = part[static_cast<int64_t>(t) * kPartFloats + kHeads * kD + h];
     const float l_raw = part[static_cast<int64_t>(t) * kPartFloats + kHeads * kD + kHeads + h];
-    const float gate = t < 32 ? a.qfull[h * kQS + kD + 32 * r + dl] : 0.0f;
+    const float gate = t < 64 ? a.qfull[h * kQS + kD + 32 * r + dl] : 0.0f;
     const datc_shape s = datc_shape_of<SP>(a);
     if (!s.valid || (FUSED && prepare_refused(pa, 1))) {
         return;
     }
     const float m_t = t < s.active ? m_raw : -INFINITY;
     const float l_t = t < s.active ? l_raw : 0.0f;
-    float mx = m_t;
-#pragma unroll
-    for (int32_t o = 32; o > 0; o >>= 1) {
-        mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    }
+    const float mx = wave_max(m_t);
     if ((t & 63) == 0) {
         wred[0][wave] = mx;
     }
@@ -576,11 +578,7 @@ __global__ __launch_bounds__(256) void datc_fold_kernel(fnkv_datc_attend_args a,
     const float M = fmaxf(fmaxf(wred[0][0], wred[0][1]), fmaxf(wred[0][2], wred[0][3]));
     const float wt = t < s.active ? expf(m_t - M) : 0.0f;
     w_of[t] = wt;
-    float lw = l_t * wt;
-#pragma unroll
-    for (int32_t o = 32; o > 0; o >>= 1) {
-        lw += __shfl_xor(lw, o, 64);
-    }
+    const float lw = wave_sum(l_t * wt);
     if ((t & 63) == 0) {
         wred[1][wave] = lw;
     }
@@ -593,19 +591,21 @@ __global__ __launch_bounds__(256) void datc_fold_kernel(fnkv_datc_attend_args a,
     }
     accs[grp][dl] = acc;
     __syncthreads();
-    if (t >= 32) {
+    if (t >= 64) { // (the first wave's second half repeats the first: the lane steps below want it whole)
         return;
     }
     const float A = ((accs[0][dl] + accs[1][dl]) + (accs[2][dl] + accs[3][dl])) +
                     ((accs[4][dl] + accs[5][dl]) + (accs[6][dl] + accs[7][dl]));
     const float y = A / L * (1.0f / (1.0f + expf(-gate)));
-    a.out[dd] = y;
     const float yv[1] = {y};
     int8_t qv[1];
     float ds[2];
     act_run<1, 32>(yv, qv, ds);
-    a.codes[dd] = qv[0];
-    if (dl == 0) {
+    if (t < 32) {
+        a.out[dd] = y;
+        a.codes[dd] = qv[0];
+    }
+    if (t == 0) {
         a.scales[2 * (h * 8 + r)] = ds[0];
         a.scales[2 * (h * 8 + r) + 1] = ds[1];
     }

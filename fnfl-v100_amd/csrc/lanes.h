@@ -1,5 +1,6 @@
 // Cross-lane steps on the VALU (DPP row moves, v_permlane16_swap / v_permlane32_swap) where a shuffle would take an LDS
-// round trip (~100 cycles each, in dependent chains of three to six). Every lane of the wave must be active.
+// round trip (~100 cycles each, in dependent chains of three to six). The lanes a step reads must be active: the group of
+// 8 or 16, or the wave.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -54,6 +55,25 @@ __device__ __forceinline__ float wave_sum(float x) {
     x += dpp_f<kDppRor + 4>(x);
     x += dpp_f<kDppRor + 2>(x);
     return x + dpp_f<kDppRor + 1>(x);
+}
+
+// max (sum, whole numbers) of x over each half of the wave
+__device__ __forceinline__ float max32(float x) {
+    x = max16(x);
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+__device__ __forceinline__ int32_t sum32(int32_t x) {
+    x = sum8(x);
+    x += dpp_i<kDppMirror>(x);
+    const auto a = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(x), static_cast<uint32_t>(x), false, false);
+    return static_cast<int32_t>(a[0] + a[1]);
+}
+// the max of x over the wave
+__device__ __forceinline__ float wave_max(float x) {
+    x = max32(x);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
 } // namespace fnkv

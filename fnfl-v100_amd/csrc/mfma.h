@@ -205,9 +205,10 @@ __device__ __forceinline__ const void * uniform_ptr(const void * p) {
 __device__ __forceinline__ rsrc_t make_rsrc(const void * base, int32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(uniform_ptr(base)), 0, bytes, 0x00020000);
 }
-// 16 B a lane at base + voff + soff into registers
+// 16 B a lane at base + voff + soff into registers (cache policy AUX, as buf_lds16's)
+template <int AUX = kStreamAux>
 __device__ __forceinline__ u32x4 buf_load16(rsrc_t r, int32_t voff, int32_t soff) {
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kStreamAux));
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, AUX));
 }
 // a wave's 64 x 16 B at base + soff + 16 lane straight into LDS at lds_base + 16 lane (cache policy AUX: the streaming
 // bit, or 0 where another wave reads the same bytes right after)

@@ -109,20 +109,13 @@ __device__ __forceinline__ uint2 pack4_f16(const float (&x)[4], float scale) {
 // exact in int32). Every lane of the run takes part; the run's first lane gets {d, s} through `ds`.
 template <int N, int WIDTH>
 __device__ __forceinline__ void act_run(const float (&y)[N], int8_t (&q)[N], float (&ds)[2]) {
-    static_assert(N * WIDTH == 32, "a run is 32 values");
+    static_assert(N * WIDTH == 32 && (WIDTH == 8 || WIDTH == 32), "a run is 32 values");
     float amax = 0.0f;
 #pragma unroll
     for (int32_t e = 0; e < N; ++e) {
         amax = fmaxf(amax, fabsf(y[e]));
     }
-    if constexpr (WIDTH == 8) {
-        amax = max8(amax);
-    } else {
-#pragma unroll
-        for (int32_t o = WIDTH / 2; o > 0; o >>= 1) {
-            amax = fmaxf(amax, __shfl_xor(amax, o, 64));
-        }
-    }
+    amax = WIDTH == 8 ? max8(amax) : max32(amax);
     const float d = amax / 127.0f;
     const float id = amax > 0.0f ? 127.0f / amax : 0.0f;
     int32_t sum = 0;
@@ -133,14 +126,7 @@ __device__ __forceinline__ void act_run(const float (&y)[N], int8_t (&q)[N], flo
         q[e] = static_cast<int8_t>(c);
         sum += c;
     }
-    if constexpr (WIDTH == 8) {
-        sum = sum8(sum);
-    } else {
-#pragma unroll
-        for (int32_t o = WIDTH / 2; o > 0; o >>= 1) {
-            sum += __shfl_xor(sum, o, 64);
-        }
-    }
+    sum = WIDTH == 8 ? sum8(sum) : sum32(sum);
     ds[0] = d;
     ds[1] = d * static_cast<float>(sum);
 }
