@@ -49,9 +49,14 @@ sparse_plan plan_sparse(const kv_pool & p, int64_t last, int32_t rows, int32_t G
     }
     pl.many = pl.n_splits < full;
     auto up16 = [](int64_t x) { return (x + 15) & ~int64_t(15); };
-    const int64_t prows = int64_t(rows) * pl.n_splits * p.h_kv() * G;
-    pl.pml_off = prows * kHeadDim * 4;
-    pl.bytes = up16(pl.pml_off + prows * 2 * 4);
+    const int64_t head_rows = int64_t(p.h_kv()) * G;
+    pl.pml_off = rows * pl.n_splits * head_rows * kHeadDim * 4;
+    // what the workspace is asked to hold: no fewer row splits than any smaller launch takes, so that one sized for a
+    // caller's largest chunk serves its smaller ones (which take more splits a row)
+    const int64_t fill = std::max<int64_t>(2 * int64_t(device_cus(p.device())) / (int64_t(p.h_kv()) * ((G + 15) / 16)),
+                                           int64_t(kSelMaxRows) * full);
+    const int64_t units = std::max<int64_t>(rows, std::min<int64_t>(int64_t(rows) * full, fill));
+    pl.bytes = up16(units * head_rows * (kHeadDim + 2) * 4);
     return pl;
 }
 

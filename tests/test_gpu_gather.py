@@ -76,3 +76,14 @@ def test_prompt_rows_at_the_split_rule(rows, hq, h_kv):
     assert err == 0 and np.isfinite(o32).all()
     assert float(np.abs(o32.astype(np.float64) - ref).max()) <= TOL
     assert np.array_equal(o16.view(np.uint16), o32.astype(np.float16).view(np.uint16))
+
+
+@pytest.mark.parametrize("hq,hkv", [(12, 1), (16, 2), (48, 1)])
+def test_prompt_workspace_serves_smaller_chunks(hq, hkv):
+    # the bytes for a caller's largest chunk hold every smaller or shallower one's partials
+    pool = fnkv.Pool(1, 4, 1, hkv)
+    rows = sorted({*range(1, 40), 100, 127, 128, 129, 255, 256, 257, 300, 511, 512, 513, 700, 1000, 2048})
+    for a, b in zip(rows, rows[1:]):
+        for pos0 in (0, 100, 2000, 40000):
+            assert 0 < pool.qsp_ws_bytes(pos0, a, hq) <= pool.qsp_ws_bytes(pos0, b, hq)
+            assert pool.qsp_ws_bytes(pos0, a, hq) <= pool.qsp_ws_bytes(pos0 + 1000, a, hq)
