@@ -45,6 +45,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <mutex>
 
 namespace fnkv {
@@ -589,7 +590,8 @@ struct pf_plan {
 };
 constexpr int32_t kPfFixed = 5;
 constexpr int32_t kPfMaxSplit = 256;
-pf_plan plan_prefill(const kv_pool & p, int64_t ctx, int32_t rows, int32_t G) {
+// (max_ws: the bytes that the splits' partials may take)
+pf_plan plan_prefill(const kv_pool & p, int64_t ctx, int32_t rows, int32_t G, int64_t max_ws = INT64_MAX) {
     pf_plan pl;
     const int32_t tok_per_wg = kPfRows / G;
     pl.row_blocks = (rows + tok_per_wg - 1) / tok_per_wg;
@@ -613,7 +615,7 @@ pf_plan plan_prefill(const kv_pool & p, int64_t ctx, int32_t rows, int32_t G) {
         const int64_t size = (max_tiles + ns - 1) / ns;
         const int64_t wgs = workgroups(size);
         const int64_t rounds = (wgs + cus - 1) / cus;
-        if (ns > least && rounds > 2) {
+        if (ns > least && (rounds > 2 || ns > max_ws / split_bytes)) {
             break; // more rounds only add fixed cost and partials
         }
         const double bytes = double(split_bytes) * double(wgs) / double(pl.row_blocks * p.h_kv());
@@ -676,8 +678,10 @@ int fnkv_attn_prefill(const fnkv_pool * pool, int32_t slot, int32_t layer, int64
     a.hq = hq;
     a.layer = layer;
     a.slot = slot;
-    fnkv::pf_plan pl = fnkv::plan_prefill(*p, ctx, rows, G);
-    if (pl.n_split > 1 && (ws == nullptr || ws_bytes < pl.ws_bytes || (reinterpret_cast<uintptr_t>(ws) & 15) != 0)) {
+    // a workspace sized for other chunks takes the best splits that it holds
+    const int64_t max_ws = ws == nullptr || (reinterpret_cast<uintptr_t>(ws) & 15) != 0 ? 0 : ws_bytes;
+    fnkv::pf_plan pl = fnkv::plan_prefill(*p, ctx, rows, G, max_ws);
+    if (pl.n_split > 1 && max_ws < pl.ws_bytes) {
         // no (or too small a) workspace: one split, written directly
         pl.n_split = 1;
         pl.split_tiles = static_cast<int32_t>((ctx + fnkv::kTileTokens - 1) / fnkv::kTileTokens);

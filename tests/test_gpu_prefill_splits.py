@@ -49,3 +49,27 @@ def test_splits_cover_every_row(depth, rows, hq, hkv, fmt):
     ref = O.attn_f64(q16.view(np.uint16), kf, vf, ctx, rows=check)
     assert cases.out_err(got.cpu().numpy()[check], ref) <= TOL
     assert cases.out_err(one.cpu().numpy()[check], ref) <= TOL
+
+
+@pytest.mark.parametrize("share", [0.2, 0.5, 0.99])
+def test_a_workspace_below_the_plans(share):
+    # a workspace sized for other chunks: the best splits that it holds, down to one
+    depth, rows, hq, hkv = 9000, 65, 16, 2
+    ctx = depth + rows
+    pool = fnkv.Pool(2, -(-ctx // 256) + 4, 1, hkv)
+    cases.scatter_ensure(pool, [0], [ctx], 77, churn=0.3)
+    k16, v16 = cases.kv_rows(77, ctx, hkv)
+    pool.append(0, 0, 0, torch.from_numpy(k16).cuda(), torch.from_numpy(v16).cuda())
+    q16 = cases.queries(77, (rows, hq, 256))
+    q = torch.from_numpy(q16).cuda()
+    got = torch.full_like(q, float("nan"))
+    need = pool.prefill_ws_bytes(ctx, rows, hq)
+    ws = torch.empty(int(need * share) // 16 * 16, dtype=torch.uint8, device="cuda")
+    guard = torch.full((1 << 20,), 0x5a, dtype=torch.uint8, device="cuda")
+    pool.prefill(0, 0, ctx, q, got, ws=ws)
+    torch.cuda.synchronize()
+    assert int((guard != 0x5a).sum()) == 0
+    (_, _, kf), (_, _, vf) = cases.decoded(O, k16, v16)
+    check = [0, 1, 32, 63, 64]
+    ref = O.attn_f64(q16.view(np.uint16), kf, vf, ctx, rows=check)
+    assert cases.out_err(got.cpu().numpy()[check], ref) <= TOL
