@@ -183,21 +183,26 @@ struct dec_plan {
     int32_t split0[FNKV_MAX_SEQS + 1] = {0};
     // the workspace: the fold state (first, at a fixed place: its words persist from launch to launch, zero), then
     // the partials
-    int64_t fold_bytes = 0, po_bytes = 0, pml_bytes = 0;
+    int64_t fold_bytes = 0, po_bytes = 0;
+    int64_t bytes = 0; // what the workspace is asked to hold (split_choice::asked)
     bool fold = false; // the stream kernel folds the splits itself (no merge launch)
 };
 
 dec_plan plan_decode(const kv_pool & p, int32_t n_seq, const int64_t * ctx, int32_t R, bool fine = true) {
     dec_plan pl;
     const int32_t cus = device_cus(p.device());
-    pl.split_tokens = choose_split_stream(n_seq, ctx, p.h_kv(), cus, (R + 15) / 16, fine);
+    const split_choice pick = choose_split_stream(n_seq, ctx, p.h_kv(), cus, (R + 15) / 16, fine);
+    pl.split_tokens = pick.cells;
+    int32_t asked = pick.asked;
     // tuning knob for measurement: FNKV_SPLIT_TOKENS (a multiple of 32 from 256 to 4,096), read once per process
     static const int32_t split_knob = env_int_once("FNKV_SPLIT_TOKENS", 0);
     if (split_knob >= kPageTokens && split_knob <= kMaxSplitPages * kPageTokens && split_knob % kTileTokens == 0) {
-        pl.split_tokens = split_knob;
+        pl.split_tokens = asked = split_knob;
     }
     pl.split0[0] = 0;
+    int64_t splits_asked = 0;
     for (int32_t i = 0; i < n_seq; ++i) {
+        splits_asked += (ctx[i] + asked - 1) / asked;
         pl.split0[i + 1] = pl.split0[i] + static_cast<int32_t>((ctx[i] + pl.split_tokens - 1) / pl.split_tokens);
     }
     // one row tile (R <= 16): the splits of a sequence stride over its tiles, so at any moment the workgroups read
@@ -207,7 +212,7 @@ dec_plan plan_decode(const kv_pool & p, int32_t n_seq, const int64_t * ctx, int3
     pl.total = pl.split0[n_seq];
     pl.fold_bytes = (int64_t(FNKV_MAX_SEQS) * p.h_kv() * kFoldWords * 4 + 255) & ~int64_t(255);
     pl.po_bytes = int64_t(pl.total) * p.h_kv() * R * kHeadDim * 4;
-    pl.pml_bytes = int64_t(pl.total) * p.h_kv() * R * 2 * 4;
+    pl.bytes = pl.fold_bytes + std::max<int64_t>(pl.total, splits_asked) * p.h_kv() * R * (kHeadDim + 2) * 4;
     // the fold waits for the other splits of its pair, so every workgroup of the launch must be resident at once:
     // one a CU (the stream kernel's LDS)
     pl.fold = fold_enabled() && int64_t(pl.total) * p.h_kv() <= cus;
@@ -352,11 +357,11 @@ int decode_launch(const fnkv_pool * pool, int32_t n_seq, const int32_t * slots, 
         }
     }
     dec_plan pl = plan_decode(*p, n_seq, ctx, R);
-    if (ws_bytes < pl.fold_bytes + pl.po_bytes + pl.pml_bytes) {
+    if (ws_bytes < pl.bytes) {
         // (a workspace sized for longer contexts can be smaller than the fine splits of short ones need)
         pl = plan_decode(*p, n_seq, ctx, R, false);
     }
-    if (ws_bytes < pl.fold_bytes + pl.po_bytes + pl.pml_bytes) {
+    if (ws_bytes < pl.bytes) {
         set_error(name + ": workspace too small");
         return FNKV_ERR_ARG;
     }
@@ -537,7 +542,7 @@ int64_t fnkv_decode_workspace_bytes(const fnkv_pool * pool, int32_t n_seq, const
     }
     const int32_t R = (hq / p->h_kv()) * T;
     const fnkv::dec_plan pl = fnkv::plan_decode(*p, n_seq, ctx, R);
-    return pl.fold_bytes + pl.po_bytes + pl.pml_bytes + 256;
+    return pl.bytes + 256;
 }
 
 void fnkv_test_decode_fold(int32_t mode, int64_t spin_ticks) {

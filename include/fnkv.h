@@ -130,7 +130,8 @@ int fnkv_export_kv8(const fnkv_pool * pool, int32_t slot, int32_t layer, int32_t
 /* The workspace a decode launch over these sequences needs (bytes; device memory the caller allocates and zeroes
  * once before its first use: its first bytes hold the counters of the launch's split-K fold, which every launch
  * leaves ready for the next, as the reference's attend workspace, attend.h:89-93). ctx[n_seq] as for
- * fnkv_attn_decode. */
+ * fnkv_attn_decode. Short contexts take finer splits than long ones and can need more: a workspace sized for longer
+ * contexts that does not hold them runs the coarser splits instead. */
 int64_t fnkv_decode_workspace_bytes(const fnkv_pool * pool, int32_t n_seq, const int64_t * ctx, int32_t T, int32_t hq);
 
 /* Dense causal attention of T query tokens of each of n_seq sequences over their pooled Q8_0 K/V of `layer`.
@@ -360,8 +361,8 @@ int64_t fnkv_prefill_workspace_bytes(const fnkv_pool * pool, int64_t ctx, int32_
  * hi + lo fp16 operands, P as hi + lo fp16 (the reference's prompt attention rounds its operands to fp16 once,
  * qsa_prompt.h:55-58; this keeps ~22 bits a product). q: fp16 [rows][hq][256], out: fp16 [rows][hq][256].
  * ws: fnkv_prefill_workspace_bytes bytes of device memory (no zeroing needed) for the key-split partials when the
- * query rows alone do not fill the device; null (or smaller): one split, no workspace. The GQA group hq / h_kv must
- * divide 256 (a workgroup's query rows). */
+ * query rows alone do not fill the device; smaller: the splits that it holds; null: one split, no workspace. The GQA
+ * group hq / h_kv must divide 256 (a workgroup's query rows). */
 int fnkv_attn_prefill(const fnkv_pool * pool, int32_t slot, int32_t layer, int64_t ctx, int32_t rows, int32_t hq,
                       float scale, const void * q, void * out, void * ws, int64_t ws_bytes, void * stream);
 
