@@ -1206,7 +1206,7 @@ def time_decode(args, torch, fnkv, cases, ctxs, T, layers, copies, fmt, steps, w
     pool.close()
 
     bytes_layer = algorithmic_bytes(ctxs, T)
-    launch_s = gpu_s / (n_steps * layers)  # one layer's attention launch (decode_kernel + merge_kernel)
+    launch_s = gpu_s / (n_steps * layers)  # one layer's attention launch (stream_kernel + the merge)
     achieved = bytes_layer / launch_s / 1e9
     return {"tokens_s": round(n * T * n_steps / wall, 3), "n_steps": n_steps, "warmup": warm * copies,
             "ms_per_step": round(wall / n_steps * 1e3, 4), "graph": not args.no_graph, "copies": copies,
