@@ -84,3 +84,21 @@ def test_walks_past_64_tiles(G, T, dev_slack, fmt):
     ctxs, hkv = [17001], 32
     q16, got, rows = launch(ctxs, T, G * hkv, hkv, 940 + G, dev_slack, fmt=fmt)
     check(q16, got, rows, ctxs, G * hkv, hkv, [0, 13, 31], fmt=fmt)
+
+
+@pytest.mark.parametrize("fmt", [fnkv.FMT_Q8_0, fnkv.FMT_KV8])
+def test_long_walks_keep_the_precision(fmt):
+    # 16,384 cells take walks of 64 tiles, 17,001 walks of 68, whose weights lie one binary place higher: the part of
+    # the error that comes from fp16's floor under the weights (most of it) halves, so the whole falls by a fifth at
+    # least; without the lead the longer walks are no closer to 64 bits than the shorter
+    hkv, T, heads = 32, 5, [0, 13, 31]
+    rel = []
+    for c in (16384, 17001):
+        q16, got, rows = launch([c], T, 8 * hkv, hkv, 960, fmt=fmt)
+        k16, v16 = (np.ascontiguousarray(x[:, heads]) for x in rows[0])
+        (_, _, kf), (_, _, vf) = (cases.decoded_kv8 if fmt == fnkv.FMT_KV8 else cases.decoded)(O, k16, v16)
+        q_heads = [8 * h + g for h in heads for g in range(8)]
+        ref = O.attn_f64(np.ascontiguousarray(q16[0][:, q_heads]).view(np.uint16), kf, vf, c)
+        rel.append(np.linalg.norm(got[0][:, q_heads].astype(np.float64) - ref) / np.linalg.norm(ref))
+    print(f"relative error: 64 tiles {rel[0]:.3e}, 68 tiles {rel[1]:.3e}")
+    assert rel[1] <= 0.8 * rel[0]
