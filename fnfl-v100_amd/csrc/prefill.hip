@@ -74,7 +74,8 @@ constexpr int32_t kPfKsc = 512;                      // the K scales in the scor
 constexpr int32_t kPfKscOff = 2 * kPfPlane;
 constexpr int32_t kPfSet = kPfKscOff + kPfKsc;       // a tile's planes: K codes, V codes, K scales
 constexpr int32_t kPfScaleRing = 4;                  // tiles' scale chunks (K then V scales, 1 KiB), a ring
-constexpr int32_t kPfPages = 2048;                   // the split's page table entries held in LDS (a split <= 512 K cells)
+constexpr int32_t kPfPages = 2048;                   // the split's page table entries held in LDS
+constexpr int32_t kPfPageTiles = (kPfPages - 1) * kTilesPerPage; // a split of at most these, wherever it starts, fits them
 constexpr int32_t kPfRegBlocks = 4;                  // q's blocks held in registers; the others' operands sit in LDS
 constexpr int32_t kPfQWave = (kBlocks - kPfRegBlocks) * kPfNT * 1024; // a wave's: [block][row tile][lane] 16 B
 constexpr int32_t kPfQOff = 2 * kPfSet + kPfScaleRing * 1024 + kPfPages * 4;
@@ -108,7 +109,9 @@ __device__ __forceinline__ void pf_load_codes(const uint8_t * tile, int32_t wave
     keep_issued();
 }
 
-__global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
+// TABLE: the page-table entries are read from the device table, tile by tile (splits that span more pages than the LDS
+// copy holds: only launches without a workspace for the plan's splits, over more than 524,032 cells)
+template <bool TABLE> __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int32_t lane = static_cast<int32_t>(threadIdx.x) & 63;
     const int32_t wave = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x) >> 6);
@@ -156,7 +159,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
     // trip on the path to its copy
     int32_t * const pages = reinterpret_cast<int32_t *>(ring_base + kPfScaleRing * 1024);
     const int32_t page0 = (ts0 * kTileTokens) >> 8;
-    const int32_t n_pages = n_tiles > 0 ? (((ts0 + n_tiles - 1) * kTileTokens) >> 8) - page0 + 1 : 0;
+    const int32_t n_pages = n_tiles > 0 && !TABLE ? (((ts0 + n_tiles - 1) * kTileTokens) >> 8) - page0 + 1 : 0;
     for (int32_t i = static_cast<int32_t>(threadIdx.x); i < n_pages; i += 64 * kPfWaves) {
         pages[i] = table[page0 + i];
     }
@@ -164,7 +167,7 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
     auto tile_ptr = [&](int32_t li) -> const uint8_t * { // the split's li-th tile (past the last: the last again)
         li = li < n_tiles ? li : n_tiles - 1;
         const int64_t tok = int64_t(ts0 + li) * kTileTokens;
-        const int32_t phys = __builtin_amdgcn_readfirstlane(pages[(tok >> 8) - page0]);
+        const int32_t phys = __builtin_amdgcn_readfirstlane(TABLE ? table[tok >> 8] : pages[(tok >> 8) - page0]);
         return layer_base + int64_t(phys) * pv.page_stride + int64_t((tok & 255) >> 5) * kTileBytes;
     };
     auto ring = [&](int32_t li) { return ring_base + (li & (kPfScaleRing - 1)) * 1024; };
@@ -448,7 +451,9 @@ __global__ __launch_bounds__(64 * kPfWaves, 1) void prefill_kernel(pf_args a) {
     for (int32_t ti = 0; ti < n_tiles; ++ti) {
         PF_T(0);
         if (wave == 0) {
-            wait_vmcnt<2>(); // tile ti + 1's scales (its two code loads may be in flight)
+            // tile ti + 1's scales (its two code loads may be in flight; TABLE: they are waited for too, since the count
+            // takes no other memory operations after the scales' copy)
+            wait_vmcnt<TABLE ? 0 : 2>();
         }
         barrier_keep_loads();
         PF_T(1);
@@ -599,8 +604,7 @@ pf_plan plan_prefill(const kv_pool & p, int64_t ctx, int32_t rows, int32_t G, in
     const int64_t cus = device_cus(p.device());
     const int64_t split_bytes = int64_t(p.h_kv()) * rows * G * (kHeadDim + 2) * 4; // one split's partials
     // a split's pages fit the kernel's LDS copy of the table
-    const int64_t page_tiles = kPfPages * kTilesPerPage - kTilesPerPage;
-    const int64_t least = std::max<int64_t>(1, (max_tiles + page_tiles - 1) / page_tiles);
+    const int64_t least = std::max<int64_t>(1, (max_tiles + kPfPageTiles - 1) / kPfPageTiles);
     const int64_t most = std::max(least, std::min<int64_t>(kPfMaxSplit, max_tiles));
     auto workgroups = [&](int64_t size) { // with tiles, at splits of `size` tiles
         int64_t n = 0;
@@ -682,7 +686,8 @@ int fnkv_attn_prefill(const fnkv_pool * pool, int32_t slot, int32_t layer, int64
     const int64_t max_ws = ws == nullptr || (reinterpret_cast<uintptr_t>(ws) & 15) != 0 ? 0 : ws_bytes;
     fnkv::pf_plan pl = fnkv::plan_prefill(*p, ctx, rows, G, max_ws);
     if (pl.n_split > 1 && max_ws < pl.ws_bytes) {
-        // no (or too small a) workspace: one split, written directly
+        // no (or too small a) workspace: one split, written directly (over the device's page table where it spans more
+        // pages than the kernel's copy holds)
         pl.n_split = 1;
         pl.split_tiles = static_cast<int32_t>((ctx + fnkv::kTileTokens - 1) / fnkv::kTileTokens);
         pl.wgs = int64_t(pl.row_blocks) * p->h_kv();
@@ -702,14 +707,21 @@ int fnkv_attn_prefill(const fnkv_pool * pool, int32_t slot, int32_t layer, int64
             int32_t cur = 0;
             (void)hipGetDevice(&cur);
             (void)hipSetDevice(dev);
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(fnkv::prefill_kernel),
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(fnkv::prefill_kernel<false>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, fnkv::kPfLds);
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(fnkv::prefill_kernel<true>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, fnkv::kPfLds);
             (void)hipGetLastError();
             (void)hipSetDevice(cur);
         });
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(fnkv::prefill_kernel, dim3(static_cast<uint32_t>(pl.wgs)), dim3(64 * fnkv::kPfWaves), fnkv::kPfLds, st, a);
+    const dim3 grid(static_cast<uint32_t>(pl.wgs)), block(64 * fnkv::kPfWaves);
+    if (pl.split_tiles > fnkv::kPfPageTiles) {
+        hipLaunchKernelGGL(fnkv::prefill_kernel<true>, grid, block, fnkv::kPfLds, st, a);
+    } else {
+        hipLaunchKernelGGL(fnkv::prefill_kernel<false>, grid, block, fnkv::kPfLds, st, a);
+    }
     if (pl.n_split > 1) {
         // a row's splits over four waves from 9 splits on (then the rows are few: a wave's chain of loads is what counts)
         const int64_t items = int64_t(p->h_kv()) * rows * G;

@@ -73,3 +73,26 @@ def test_a_workspace_below_the_plans(share):
     check = [0, 1, 32, 63, 64]
     ref = O.attn_f64(q16.view(np.uint16), kf, vf, ctx, rows=check)
     assert cases.out_err(got.cpu().numpy()[check], ref) <= TOL
+
+
+@pytest.mark.parametrize("pages", [2047, 2050])
+def test_one_split_past_the_page_copy(pages):
+    # without a workspace a chunk's keys are one split: up to 2,047 pages its page numbers sit in LDS (2,048 entries),
+    # past them the launch reads the device's table
+    rows, hq = 5, 8
+    ctx = pages * 256 - 100
+    pool = fnkv.Pool(2, pages + 4, 1, 1)
+    cases.scatter_ensure(pool, [0], [ctx], 91)
+    k16, v16 = cases.kv_rows(91, ctx, 1)
+    pool.append(0, 0, 0, torch.from_numpy(k16).cuda(), torch.from_numpy(v16).cuda())
+    q16 = cases.queries(91, (rows, hq, 256))
+    q = torch.from_numpy(q16).cuda()
+    got, one = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    pool.prefill(0, 0, ctx, q, got)
+    pool.prefill(0, 0, ctx, q, one, ws=False)
+    torch.cuda.synchronize()
+    (_, _, kf), (_, _, vf) = cases.decoded(O, k16, v16)
+    ref = O.attn_f64(q16.view(np.uint16), kf, vf, ctx, rows=[0, 4])
+    assert cases.out_err(got.cpu().numpy()[[0, 4]], ref) <= TOL
+    assert cases.out_err(one.cpu().numpy()[[0, 4]], ref) <= TOL
+    assert cases.out_err(one.cpu().numpy(), got.cpu().numpy()) <= 2 * TOL
