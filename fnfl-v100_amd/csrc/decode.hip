@@ -188,16 +188,27 @@ struct dec_plan {
     bool fold = false; // the stream kernel folds the splits itself (no merge launch)
 };
 
-dec_plan plan_decode(const kv_pool & p, int32_t n_seq, const int64_t * ctx, int32_t R, bool fine = true) {
+int64_t fold_region_bytes(const kv_pool & p) {
+    return (int64_t(FNKV_MAX_SEQS) * p.h_kv() * kFoldWords * 4 + 255) & ~int64_t(255);
+}
+// one split's partials (every KV head's R rows)
+int64_t split_bytes(const kv_pool & p, int32_t R) { return int64_t(p.h_kv()) * R * (kHeadDim + 2) * 4; }
+
+// max_splits: the partials that the workspace holds (then nothing more is asked of it); total 0 if no size makes so few
+dec_plan plan_decode(const kv_pool & p, int32_t n_seq, const int64_t * ctx, int32_t R, bool fine = true,
+                     int64_t max_splits = kAnySplits) {
     dec_plan pl;
     const int32_t cus = device_cus(p.device());
-    const split_choice pick = choose_split_stream(n_seq, ctx, p.h_kv(), cus, (R + 15) / 16, fine);
+    const split_choice pick = choose_split_stream(n_seq, ctx, p.h_kv(), cus, (R + 15) / 16, fine, max_splits);
     pl.split_tokens = pick.cells;
-    int32_t asked = pick.asked;
+    int32_t asked = max_splits < kAnySplits ? pick.cells : pick.asked;
     // tuning knob for measurement: FNKV_SPLIT_TOKENS (a multiple of 32 from 256 to 4,096), read once per process
     static const int32_t split_knob = env_int_once("FNKV_SPLIT_TOKENS", 0);
     if (split_knob >= kPageTokens && split_knob <= kMaxSplitPages * kPageTokens && split_knob % kTileTokens == 0) {
         pl.split_tokens = asked = split_knob;
+    }
+    if (pl.split_tokens == 0) {
+        return pl;
     }
     pl.split0[0] = 0;
     int64_t splits_asked = 0;
@@ -210,9 +221,9 @@ dec_plan plan_decode(const kv_pool & p, int32_t n_seq, const int64_t * ctx, int3
     // decode_launch); more rows: contiguous splits
     pl.strided = R <= 16 ? 1 : 0;
     pl.total = pl.split0[n_seq];
-    pl.fold_bytes = (int64_t(FNKV_MAX_SEQS) * p.h_kv() * kFoldWords * 4 + 255) & ~int64_t(255);
+    pl.fold_bytes = fold_region_bytes(p);
     pl.po_bytes = int64_t(pl.total) * p.h_kv() * R * kHeadDim * 4;
-    pl.bytes = pl.fold_bytes + std::max<int64_t>(pl.total, splits_asked) * p.h_kv() * R * (kHeadDim + 2) * 4;
+    pl.bytes = pl.fold_bytes + std::max<int64_t>(pl.total, splits_asked) * split_bytes(p, R);
     // the fold waits for the other splits of its pair, so every workgroup of the launch must be resident at once:
     // one a CU (the stream kernel's LDS)
     pl.fold = fold_enabled() && int64_t(pl.total) * p.h_kv() <= cus;
@@ -360,6 +371,18 @@ int decode_launch(const fnkv_pool * pool, int32_t n_seq, const int32_t * slots, 
     if (ws_bytes < pl.bytes) {
         // (a workspace sized for longer contexts can be smaller than the fine splits of short ones need)
         pl = plan_decode(*p, n_seq, ctx, R, false);
+    }
+    if (ws_bytes < pl.bytes) {
+        // The rule's split count falls where the contexts outgrow one round of workgroups at one size and the next larger
+        // size takes them in one (2 KV heads: 131,041 cells 128 splits, 140,000 cells 110), so a workspace sized for
+        // deeper contexts can hold fewer splits than a shorter call's. It holds half a round's at least, and the deeper
+        // call's size makes no more splits of the shorter contexts: the best of the sizes that it holds. (A workspace
+        // below that and below the call's own stays refused.)
+        const int64_t holds = (ws_bytes - fold_region_bytes(*p)) / split_bytes(*p, R);
+        if (holds >= std::max(1, device_cus(p->device()) / (2 * p->h_kv()))) {
+            const dec_plan held = plan_decode(*p, n_seq, ctx, R, false, holds);
+            pl = held.total > 0 ? held : pl;
+        }
     }
     if (ws_bytes < pl.bytes) {
         set_error(name + ": workspace too small");

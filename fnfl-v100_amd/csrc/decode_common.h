@@ -258,15 +258,18 @@ struct fused_prep; // gather.h
 void launch_merge(const merge_args & m, hipStream_t st);
 // host: the dense launch's one-stream-a-wave kernel for NT = 1 .. 3 row tiles (stream.hip)
 void launch_stream(int32_t device, int32_t NT, dim3 grid, const dec_args & a, hipStream_t st);
-// the split size (cells) of a dense launch run by the stream kernel with NT row tiles; fine: kFineSplit is allowed
+// the split size (cells) of a dense launch run by the stream kernel with NT row tiles; fine: kFineSplit is allowed;
+// max_splits: at most this many splits
 constexpr int32_t kFineSplit = 128;
+constexpr int64_t kAnySplits = int64_t(1) << 40;
 struct split_choice {
     int32_t cells = 0; // a split's
     // the best split of at most 64 tiles: the workspace asked for holds its partials too, so a launch that takes longer
     // splits is refused by the same workspaces
     int32_t asked = 0;
 };
-split_choice choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_kv, int32_t cus, int32_t NT, bool fine);
+split_choice choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_kv, int32_t cus, int32_t NT, bool fine,
+                                 int64_t max_splits = kAnySplits);
 // a launch's depth read from device memory (the reference's depth word, attend.h:108): depth + T <= max_cells or
 // the launch writes nothing and ORs FNKV_DEV_ERR_DEPTH into *err
 struct dev_depth {

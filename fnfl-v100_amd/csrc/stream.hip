@@ -944,7 +944,9 @@ __global__ __launch_bounds__(512, 1) void stream_kernel(dec_args a) {
 // partial's write, counted as three tiles); larger splits (fewer partials) win ties. The longest split is what its
 // waves' page registers hold: a bound just past a round's 2,048-cell splits (262,401 cells) would otherwise take a
 // second round of half-size splits, 83.0 against 93.5 us a layer at T = 5.
-split_choice choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_kv, int32_t cus, int32_t NT, bool fine) {
+// max_splits: sizes that make more are passed over (cells 0: every size does).
+split_choice choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_kv, int32_t cus, int32_t NT, bool fine,
+                                 int64_t max_splits) {
     int64_t tiles[FNKV_MAX_SEQS];
     for (int32_t i = 0; i < n_seq; ++i) {
         tiles[i] = (ctx[i] + kTileTokens - 1) / kTileTokens;
@@ -960,10 +962,14 @@ split_choice choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_k
     };
     // sizes between two multiples of the streams' tiles cost what the upper one does and take more workgroups
     const int32_t streams = NT == 3 ? stream_shape<3>::STREAMS : stream_shape<1>::STREAMS;
-    split_choice pick = {kPageTokens, kPageTokens};
+    split_choice pick;
     int64_t best_cost = INT64_MAX;
     for (int32_t t = kPageTokens / kTileTokens; t <= kMaxSplitPages * kPageTokens / kTileTokens; t += streams) {
-        const int64_t rounds = (workgroups(static_cast<uint32_t>(t)) + cus - 1) / cus;
+        const int64_t wgs = workgroups(static_cast<uint32_t>(t));
+        if (wgs > max_splits * h_kv) {
+            continue;
+        }
+        const int64_t rounds = (wgs + cus - 1) / cus;
         const int64_t cost = rounds * (t / streams + 3);
         if (cost <= best_cost) {
             best_cost = cost;

@@ -130,8 +130,9 @@ int fnkv_export_kv8(const fnkv_pool * pool, int32_t slot, int32_t layer, int32_t
 /* The workspace a decode launch over these sequences needs (bytes; device memory the caller allocates and zeroes
  * once before its first use: its first bytes hold the counters of the launch's split-K fold, which every launch
  * leaves ready for the next, as the reference's attend workspace, attend.h:89-93). ctx[n_seq] as for
- * fnkv_attn_decode. Short contexts take finer splits than long ones and can need more: a workspace sized for longer
- * contexts that does not hold them runs the coarser splits instead. */
+ * fnkv_attn_decode. Shorter contexts can take more splits than longer ones: a workspace sized for the deepest contexts,
+ * the most sequences and the largest T (of one hq) serves every smaller call, with coarser splits where it holds fewer
+ * than the call's own size gives. */
 int64_t fnkv_decode_workspace_bytes(const fnkv_pool * pool, int32_t n_seq, const int64_t * ctx, int32_t T, int32_t hq);
 
 /* Dense causal attention of T query tokens of each of n_seq sequences over their pooled Q8_0 K/V of `layer`.

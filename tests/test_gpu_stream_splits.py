@@ -86,6 +86,38 @@ def test_walks_past_64_tiles(G, T, dev_slack, fmt):
     check(q16, got, rows, ctxs, G * hkv, hkv, [0, 13, 31], fmt=fmt)
 
 
+@pytest.mark.parametrize("deep,T_deep", [([66000], 1), ([140000], 1), ([140000], 5), ([200000], 3),
+                                         ([100000, 70000, 3000], 3)])
+def test_a_workspace_for_deeper_contexts_serves_shorter_ones(deep, T_deep):
+    # the rule's split count falls where larger splits come to fit one round of workgroups: the workspace sized for the
+    # deepest contexts and largest step runs every shorter call, as far from fp64 as with its own workspace
+    hq, hkv, layers = 16, 2, 1
+    pool = fnkv.Pool(len(deep) + 1, sum(-(-c // 256) for c in deep) + 8, layers, hkv)
+    for s, c in enumerate(deep):
+        assert pool.ensure(s, c)[0] == 0
+        g = torch.Generator(device="cuda").manual_seed(970 + s)
+        k, v = (torch.randn((c, hkv, 256), generator=g, device="cuda").half() for _ in range(2))
+        pool.append(s, 0, 0, k, v)
+    ws = torch.zeros(pool.decode_ws_bytes(deep, T_deep, hq), dtype=torch.uint8, device="cuda")
+    calls = [[c] for c in range(T_deep, deep[0], 6007)]
+    calls += [[c] for c in (22017, 32768, 33000, 65505, 98305, 131041, 131072, 196577) if c < deep[0]]
+    calls += [[max(T_deep, int(c * x)) for c in deep] for x in (0.999, 0.95, 0.7, 0.51, 0.3, 0.1)]
+    smaller = 0
+    for ctxs in calls:
+        for T in {1, T_deep}:
+            n = pool.decode_ws_bytes(ctxs, T, hq)
+            q = torch.from_numpy(cases.queries(971, (len(ctxs), T, hq, 256))).cuda()
+            got, own = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+            slots = list(range(len(ctxs)))
+            pool.decode(slots, ctxs, T, 0, q, got, ws)
+            pool.decode(slots, ctxs, T, 0, q, own, torch.zeros(n, dtype=torch.uint8, device="cuda"))
+            torch.cuda.synchronize()
+            smaller += n > ws.numel()
+            assert float((got.float() - own.float()).abs().max()) <= 2 * TOL, (ctxs, T)
+    print(f"{smaller} of {2 * len(calls)} calls ask for more than the workspace")
+    assert smaller > 0
+
+
 @pytest.mark.parametrize("fmt", [fnkv.FMT_Q8_0, fnkv.FMT_KV8])
 def test_long_walks_keep_the_precision(fmt):
     # 16,384 cells take walks of 64 tiles, 17,001 walks of 68, whose weights lie one binary place higher: the part of
