@@ -461,13 +461,14 @@ __device__ void fold_splits(const dec_args & a, int32_t s, int32_t kvh, int32_t 
             }
         }
         const uint64_t b = __ballot(take);
-        if (tid == 0) {
+        if (tid == 0) { // (up to FNKV_MAX_ROWS rows: more than a word's)
             shared_word[1] = static_cast<uint32_t>(b);
+            shared_word[2] = static_cast<uint32_t>(b >> 32);
         }
     }
     __syncthreads();
-    for (uint32_t m = shared_word[1]; m != 0; m &= m - 1) {
-        const int32_t r = __builtin_ctz(m);
+    for (uint64_t m = (uint64_t(shared_word[2]) << 32) | shared_word[1]; m != 0; m &= m - 1) {
+        const int32_t r = __builtin_ctzll(m);
         fold_rows<THREADS>(a, s, kvh, r % n, n, 1u << (r / n), smem);
     }
 }

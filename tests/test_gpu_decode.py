@@ -145,6 +145,28 @@ def test_fold_fallback_and_reused_workspace_bitwise():
     assert np.all(words[:, 0] % 1024 == 0) and words[:, 0].max() > 0
 
 
+@pytest.mark.parametrize("T,ctx", [(5, 9000), (6, 30000), (3, 700)])
+def test_fold_of_given_up_rows_covers_every_row(T, ctx):
+    # up to 48 rows a KV head: with the wait bound at zero the last split to arrive folds every row given up, those past
+    # the 32nd too, bitwise the fold's outputs (the outputs start as NaN)
+    st = Setup([ctx], seed=6)
+    q = torch.from_numpy(cases.queries(6, (1, T, HQ, 256))).cuda()
+    ws = torch.zeros(st.pool.decode_ws_bytes([ctx], T, HQ), dtype=torch.uint8, device="cuda")
+    outs = []
+    for spin in (-1, 0, 0):
+        fnkv.lib().fnkv_test_decode_fold(1, spin)
+        try:
+            out = torch.full_like(q, float("nan"))
+            st.pool.decode(st.slots, [ctx], T, 0, q, out, ws)
+            torch.cuda.synchronize()
+        finally:
+            fnkv.lib().fnkv_test_decode_fold(-1, -1)
+        outs.append(out)
+    assert bool(torch.isfinite(outs[0]).all())
+    for o in outs[1:]:
+        assert torch.equal(o.view(torch.int16), outs[0].view(torch.int16))
+
+
 def test_layers_are_separate():
     st = Setup([1500, 600], seed=4, layers=3)
     q16 = cases.queries(4, (2, 1, HQ, 256))
