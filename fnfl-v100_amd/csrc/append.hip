@@ -19,7 +19,8 @@ namespace fnkv {
 // aligned positions 4 g .. 4 g + 3 that the rows touch (the four cells' bytes of one value are adjacent in the V
 // layout, so each lane stores a dword a value; a quad the rows cover in part writes only its own cells).
 // pos_dev set: the first position is the device word *pos_dev, read by the launch; a position outside
-// 0 .. max_cells - rows writes nothing (the launch that reads the rows reports it)
+// 0 .. max_cells - rows writes nothing (the launch that reads the rows reports it). A cell of an unmapped page is not
+// written either
 template <bool F32>
 __global__ __launch_bounds__(256) void append_kernel(pool_view pv, int32_t slot, int32_t layer, int64_t pos0,
                                                      int32_t rows, const void * __restrict__ kin,
@@ -46,8 +47,10 @@ __global__ __launch_bounds__(256) void append_kernel(pool_view pv, int32_t slot,
             load4<false>(static_cast<const uint16_t *>(kin) + src, lane, x);
         }
         const int64_t pos = pos0 + row;
-        quantize_store_fmt(x, lane, tile_of(pv, table, layer, head, pos), static_cast<int32_t>(pos & 31), 0,
-                           pv.format);
+        if (page_mapped(table, pos)) {
+            quantize_store_fmt(x, lane, tile_of(pv, table, layer, head, pos), static_cast<int32_t>(pos & 31), 0,
+                               pv.format);
+        }
         return;
     }
     const int64_t vw = w - k_waves;
@@ -75,7 +78,9 @@ __global__ __launch_bounds__(256) void append_kernel(pool_view pv, int32_t slot,
             quantize_fmt(x, pv.format, packed[i], sbits[i]);
         }
     }
-    store_v_quad(packed, sbits, valid, lane, tile_of(pv, table, layer, head, p0), static_cast<int32_t>(p0 & 31));
+    if (page_mapped(table, p0)) {
+        store_v_quad(packed, sbits, valid, lane, tile_of(pv, table, layer, head, p0), static_cast<int32_t>(p0 & 31));
+    }
 }
 
 // one wave a cell: its 8 blocks of (layer, head, kv) as 8 x 34 bytes of block_q8_0

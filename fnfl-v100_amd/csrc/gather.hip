@@ -5,7 +5,8 @@
 // attend.cu:405-421, and its prompt form, qsa_prompt_attn.cu:229-436): row z of a launch sits at position q = depth + z
 // and attends to the cells of its body's K = min((q + 1) / 4, 512) ascending 4-cell blocks and to its tail cells
 // 4 ((q + 1) / 4) .. q, with the decoded Q8_0 / KV8 cells, fp32 scores, softmax statistics and accumulators. Block IDs
-// outside the row's whole blocks, and an ID equal to the one before it, are ignored.
+// outside the row's whole blocks, and an ID equal to the one before it, are ignored. A row that selects a block of an
+// unmapped page (a slot trimmed under a captured launch, outside the contract) gets no output.
 //
 // How (MI355X):
 //   * The pool's tiles hold 32 cells, a selection picks 4-cell blocks: where a selection scatters, reading whole tiles
@@ -132,9 +133,9 @@ __device__ __forceinline__ void gather_scores(const u32x4 (&kw)[8], const uint8_
 }
 
 // The row's new cells that this workgroup reads (bit c: cell depth + c) or owns: quantized and written before its
-// block loads (several workgroups may write one cell: the same bytes). Prepared rows (fp): K = the F32 RMS norm and
-// IMROPE of kv_k's row c (the row's own cell z from own_x / own_g, loaded early, at the pairs' angles rp), V = kv_v's row
-// c; else one row's k_new / v_new.
+// block loads (several workgroups may write one cell: the same bytes; a cell of an unmapped page is not written).
+// Prepared rows (fp): K = the F32 RMS norm and IMROPE of kv_k's row c (the row's own cell z from own_x / own_g, loaded
+// early, at the pairs' angles rp), V = kv_v's row c; else one row's k_new / v_new.
 __device__ __forceinline__ void gather_append(const gather_args & a, int32_t kvh, int32_t z, int64_t depth,
                                               uint32_t cells, bool own, const rope_pairs & rp,
                                               float4 own_x, float4 own_g, int32_t wave, int32_t lane) {
@@ -170,8 +171,10 @@ __device__ __forceinline__ void gather_append(const gather_args & a, int32_t kvh
         } else {
             load4<true>(a.fp.kv_v + src, lane, x);
         }
-        quantize_store_fmt(x, lane, tile_of(pv, a.table, a.layer, kvh, pos), static_cast<int32_t>(pos & 31), kv,
-                           pv.format);
+        if (__builtin_expect(page_mapped(a.table, pos), 1)) {
+            quantize_store_fmt(x, lane, tile_of(pv, a.table, a.layer, kvh, pos), static_cast<int32_t>(pos & 31), kv,
+                               pv.format);
+        }
     }
 }
 
@@ -328,9 +331,11 @@ __global__ __launch_bounds__(64 * kW, MANY ? 2 : 1) void gather_kernel(gather_ar
     uint8_t * const slot = smem + wave * kGatherSlot;
     uint32_t * const codes = reinterpret_cast<uint32_t *>(slot + 2048);
     uint8_t * const counts = slot + 2048 + 64 * kMaxRegs * 4;
+    bool hole = false; // a selected block of an unmapped page: page 0 is read in its place, and the row gets no output
 #pragma unroll
     for (int32_t m = 0; m < M; ++m) {
         const int32_t phys = page[m] >= 0 ? page[m] : 0;
+        hole = hole || (good[m] && page[m] < 0);
         good[m] = good[m] && page[m] >= 0;
         const uint32_t kib = static_cast<uint32_t>(phys) * static_cast<uint32_t>(a.pv.h_kv * kPageKib) +
                              static_cast<uint32_t>((id[m] >> 3) & 7) * kTileKib;
@@ -423,7 +428,8 @@ __global__ __launch_bounds__(64 * kW, MANY ? 2 : 1) void gather_kernel(gather_ar
 
     floatx4 acc[16];
     floatx4 lv = {0.0f, 0.0f, 0.0f, 0.0f}; // sum_t P[t][row] s_v[t][b]: lane (row j, qg) holds b = 4 qg + r
-    float m_run = kNegInf, l_run = 0.0f;
+    float m_run = __any(hole) ? __builtin_nanf("") : kNegInf; // (a NaN stays one: the folds write nothing then)
+    float l_run = 0.0f;
 #pragma unroll
     for (int m = 0; m < 16; ++m) {
         acc[m] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -542,6 +548,9 @@ __global__ __launch_bounds__(64 * kW, MANY ? 2 : 1) void gather_kernel(gather_ar
     if (qg == 0) {
         *reinterpret_cast<float2 *>(mine + 16 * kGatherOS + 2 * j) = float2{m_run, l_run};
     }
+    if (__builtin_expect(m_run != m_run, 0) && a.err != nullptr && lane == 0) {
+        atomicOr(a.err, FNKV_DEV_ERR_DEPTH);
+    }
     __syncthreads();
     // thread -> (row, 4 values): a wave a row, its 64 lanes the row's 256 values
     const int32_t c0 = lane * 4;
@@ -557,7 +566,7 @@ __global__ __launch_bounds__(64 * kW, MANY ? 2 : 1) void gather_kernel(gather_ar
 #pragma unroll
         for (int w = 0; w < kW; ++w) {
             ml[w] = *reinterpret_cast<const float2 *>(slots + w * (kGatherSlot / 4) + 16 * kGatherOS + 2 * r);
-            Mr = fmaxf(Mr, ml[w].x);
+            Mr = __builtin_elementwise_maximum(Mr, ml[w].x); // (a NaN stays one)
         }
         const float Mu = Mr == kNegInf ? 0.0f : Mr;
         float L = 0.0f;
@@ -574,7 +583,9 @@ __global__ __launch_bounds__(64 * kW, MANY ? 2 : 1) void gather_kernel(gather_ar
         }
         const int64_t row = int64_t(z) * a.hq + head0 + r;
         if (a.n_splits == 1) {
-            finish4(a.fin, row, c0, sum, L, gates[i]);
+            if (__builtin_expect(Mr == Mr, 1)) { // (uniform: a wave a row)
+                finish4(a.fin, row, c0, sum, L, gates[i]);
+            }
         } else {
             const int64_t prow = ((int64_t(z) * a.n_splits + split) * a.pv.h_kv + kvh) * a.G + 16 * rt + r;
             *reinterpret_cast<floatx4 *>(a.po + prow * kHeadDim + c0) = sum;

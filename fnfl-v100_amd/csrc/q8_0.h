@@ -31,6 +31,10 @@ __device__ __forceinline__ uint8_t * tile_of(const pool_view & pv, const int32_t
            int64_t((pos & 255) >> 5) * kTileBytes;
 }
 
+// position pos's page is mapped (-1 in the table: the slot was trimmed under a captured launch, outside the contract; a
+// write through that entry would land before the layer's plane)
+__device__ __forceinline__ bool page_mapped(const int32_t * table_row, int64_t pos) { return table_row[pos >> 8] >= 0; }
+
 // load this lane's 4 values of a 256-value row (fp16 or fp32) as fp32
 template <bool F32> __device__ __forceinline__ void load4(const void * row, int32_t lane, float (&x)[4]) {
     if (F32) {

@@ -88,6 +88,9 @@ __global__ __launch_bounds__(64) void qsa_prepare_kernel(qsa_prep_args a) {
         reinterpret_cast<float4 *>(a.k_f32 + o)[lane] = make_float4(y[0], y[1], y[2], y[3]);
     }
     const int64_t pos = a.depth + t;
+    if (!page_mapped(a.table, pos)) {
+        return; // (the attention's launch reports what the rows select there)
+    }
     uint8_t * tile = tile_of(a.pv, a.table, a.layer, kvh, pos);
     quantize_store_fmt(y, lane, tile, static_cast<int32_t>(pos & 31), 0, a.pv.format);
     float v[4];

@@ -55,6 +55,9 @@ __global__ __launch_bounds__(64) void qsp_kv_kernel(qsp_args a) {
     rope_angle(s, c, qsp_pos(a, t, lane), a.theta_scale, lane);
     norm_rope_apply(y, x, g, rope_pairs_of(s, c, lane), lane);
     const int64_t pos = int64_t(a.pos0) + t;
+    if (!page_mapped(a.table, pos)) {
+        return;
+    }
     uint8_t * tile = tile_of(a.pv, a.table, a.layer, kvh, pos);
     quantize_store_fmt(y, lane, tile, static_cast<int32_t>(pos & 31), 0, a.pv.format);
     float v[4];

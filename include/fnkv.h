@@ -218,7 +218,9 @@ int fnkv_attn_sparse(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_
  * max_cells (host) bounds depth + T, fixes the plan (workspace: fnkv_sparse_workspace_bytes(pool, max_cells - T, T,
  * hq)) and must not exceed the slot's mapped cells. A depth with depth + T beyond max_cells (or below 0) writes
  * nothing — no new cells, no out rows — and ORs FNKV_DEV_ERR_DEPTH into *err (device, caller-cleared). The body's
- * layout follows the depth read. */
+ * layout follows the depth read. The slot must stay mapped up to max_cells while a captured launch may run; a launch
+ * that nevertheless finds an unmapped page writes no new cell there, writes no out of a row that selects a block of it
+ * and ORs FNKV_DEV_ERR_DEPTH into *err for such a row (fnkv_attend likewise). */
 int fnkv_attn_sparse_dev(const fnkv_pool * pool, int32_t slot, const int32_t * depth, int64_t max_cells, int32_t T,
                          int32_t layer, int32_t hq, float scale, const void * q, const void * body,
                          const void * offsets, const void * k_new, const void * v_new, int32_t new_dtype, void * out,

@@ -250,6 +250,54 @@ def test_replay_after_trim_reads_no_unmapped_page(T):
         err.zero_()
 
 
+@pytest.mark.parametrize("form,T", [("sparse", 1), ("sparse", 3), ("attend", 1), ("attend", 3), ("attend32", 2)])
+def test_sparse_replay_after_trim_writes_nothing(form, T):
+    # The same for the sparse launches (new cells written by the launch, by an append before it, by the launch that
+    # prepares its rows, by a prepare before it): rows that select blocks past the trimmed end get no output, the error
+    # word its bit. The new cells' pages are unmapped, so none is written: entry -1 of layer 1 would be layer 0's last
+    # physical page, which the other slot holds.
+    depth, hkv = 3000, 1
+    hq = 32 if form == "attend32" else 12
+    bound, n_pages = depth + T, 20
+    pool = fnkv.Pool(2, n_pages, 2, hkv)
+    assert pool.ensure(0, bound)[0] == 0
+    assert pool.ensure(1, (n_pages - pool.mapped_cells(0) // 256) * 256)[0] == 0
+    assert n_pages - 1 in [pool.table(1)[i] for i in range(pool.mapped_cells(1) // 256)]
+    k16, v16 = cases.kv_rows(19, depth, hkv)
+    pool.append(0, 1, 0, torch.from_numpy(k16).cuda(), torch.from_numpy(v16).cuda())
+    if form == "sparse":
+        words, o, _ = O.qsa_body(depth, T, 23)
+        body, offs = torch.from_numpy(words.view(np.int32)).cuda(), torch.from_numpy(o).cuda()
+        q = torch.from_numpy(cases.queries(19, (T, hq, D))).cuda()
+        kn, vn = (torch.from_numpy(x).cuda() for x in cases.kv_rows(20, T, hkv))
+        out = torch.full_like(q, 7.0)
+        depth_dev = torch.tensor([depth], dtype=torch.int32, device="cuda")
+        err = torch.zeros(1, dtype=torch.int32, device="cuda")
+        ws = torch.empty(pool.sparse_ws_bytes(depth, T, hq), dtype=torch.uint8, device="cuda")
+        g = capture(lambda: pool.sparse_dev(0, depth_dev, bound, 1, q, body, offs, out, ws, err, k_new=kn, v_new=vn))
+    else:
+        c = AttendCase(pool, 0, T, hq, hkv, bound, seed=24)
+        c.args.layer = 1
+        c.stage(depth, 0)
+        out, err = c.out, c.err
+        g = capture(lambda: fnkv.attend(T, c.args))
+    g.replay()
+    torch.cuda.synchronize()
+    assert err.item() == 0 and bool(torch.isfinite(out).all()) and not bool((out == 7.0).all())
+    other = [pool.export(1, layer, 0, kv, 0, pool.mapped_cells(1)).cpu() for layer in range(2) for kv in range(2)]
+    assert pool.trim(0, 1024) == 0
+    kept = [pool.export(0, 1, 0, kv, 0, 1024).cpu() for kv in range(2)]
+    for _ in range(2):
+        out.fill_(7.0)
+        err.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert err.item() == fnkv.DEV_ERR_DEPTH and bool((out == 7.0).all())
+    again = [pool.export(1, layer, 0, kv, 0, pool.mapped_cells(1)).cpu() for layer in range(2) for kv in range(2)]
+    assert all(torch.equal(x, y) for x, y in zip(other, again))
+    assert all(torch.equal(x, pool.export(0, 1, 0, kv, 0, 1024).cpu()) for kv, x in enumerate(kept))
+
+
 def test_decode_dev_host_refusals_enqueue_nothing():
     L = DecodeLoop([600], 1, 1, seed=2)
     q = torch.zeros((1, 1, HQ, D), dtype=torch.float16, device="cuda")
