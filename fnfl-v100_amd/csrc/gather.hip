@@ -16,9 +16,9 @@
 //     v_mfma_f32_16x16x32_f16 reads (K: 8 loads of 16 B; V: 16 of 12 B, of which 8 are its cells'), and the scores, the
 //     softmax and PV run on the virtual tile as on a stored one. Entry e of the body is cell group e of virtual tile
 //     e / 8, so no workgroup builds a list: a lane's block is one body word and one page-table word.
-//   * A workgroup of 4 waves (one a SIMD; two workgroups a CU) owns (row, up to 16 query heads of a KV head, split):
+//   * A workgroup of 4 waves (one a SIMD; two workgroups a CU for prompt rows) owns (row, up to 16 query heads of a KV head, split):
 //     wave w of split s takes virtual tiles 4 s + w, + 4 n_splits, ... Decode rows launch enough splits for one tile a
-//     wave (at most 17 splits of a row's 65 tiles); prompt rows split only while the rows alone do not fill the device,
+//     wave (at most 17 splits of a row's 65 tiles) where those are at most one workgroup a CU; prompt rows split only while the rows alone do not fill the device,
 //     and a row of one split is finished here, without partials or a merge.
 //   * A tile's K and scales are requested while the previous tile is in its softmax and PV, its V while the next
 //     scores run; every block of the wave's tiles is resolved (body word, then page) before the first.
@@ -179,9 +179,10 @@ __device__ __forceinline__ void gather_append(const gather_args & a, int32_t kvh
 }
 
 // KV8: the pool's group-64 format. QLO: q as fp16 hi + lo, exact codes and 6 more bits of P (the attn::attend calls).
-// MANY: a wave may take several tiles (prompt rows); else at most one.
+// MANY: a wave may take several tiles (prompt rows, and decode rows of many KV heads); else at most one. Two workgroups a
+// CU fit the LDS without QLO, and the registers of MANY.
 template <bool KV8, bool QLO, bool MANY>
-__global__ __launch_bounds__(64 * kW, MANY ? 2 : 1) void gather_kernel(gather_args a) {
+__global__ __launch_bounds__(64 * kW, MANY && !QLO ? 2 : 1) void gather_kernel(gather_args a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int32_t lane = static_cast<int32_t>(threadIdx.x) & 63;
     const int32_t wave = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x) >> 6);
@@ -343,14 +344,18 @@ __global__ __launch_bounds__(64 * kW, MANY ? 2 : 1) void gather_kernel(gather_ar
         counts[64 * m + lane] = static_cast<uint8_t>(!good[m] ? 0 : id[m] == sel.n_vis ? sel.tail : 4);
     }
 
-    // New cells (decode rows; one tile a wave): the ones whose block this workgroup reads, and the row's own cell by
-    // its owner: the split that holds the tail entry, or split 0 when the row has no tail
-    const bool writes = !MANY && (a.k_new != nullptr || a.fp.kv_k != nullptr);
+    // New cells (decode rows; the form of prompt rows has none): the ones whose block this workgroup reads, and the row's
+    // own cell by its owner: the split that holds the tail entry, or split 0 when the row has no tail
+    const bool writes = (!MANY || QLO) && (a.k_new != nullptr || a.fp.kv_k != nullptr);
     uint32_t * const seen = reinterpret_cast<uint32_t *>(smem + gather_lds(QLO) - 64); // a word a wave
     if (writes) {
         uint32_t mine = 0;
         for (int32_t c = 0; c <= z; ++c) {
-            const bool hit = good[0] && id[0] == static_cast<int32_t>((depth + c) >> 2);
+            bool hit = false;
+#pragma unroll
+            for (int32_t m = 0; m < M; ++m) {
+                hit = hit || (good[m] && id[m] == static_cast<int32_t>((depth + c) >> 2));
+            }
             mine |= __any(hit) ? 1u << c : 0u;
         }
         if (lane == 0) {
@@ -364,7 +369,11 @@ __global__ __launch_bounds__(64 * kW, MANY ? 2 : 1) void gather_kernel(gather_ar
         for (int w = 0; w < kW; ++w) {
             cells |= seen[w];
         }
-        const bool own = rt == 0 && (sel.tail != 0 ? (sel.K >> 3) / kW : 0) == split;
+        int32_t owner = sel.tail != 0 ? (sel.K >> 3) / kW : 0;
+        if constexpr (MANY) {
+            owner %= a.n_splits;
+        }
+        const bool own = rt == 0 && owner == split;
         cells |= own ? 1u << z : 0u;
         if (cells != 0) { // uniform in the workgroup
             gather_append(a, kvh, z, depth, cells, own, rp, own_x, own_g, wave, lane);
@@ -620,6 +629,8 @@ void launch_gather(int32_t device, const gather_args & a, hipStream_t st) {
             set_gather_attr<true, true, false>();
             set_gather_attr<false, false, true>();
             set_gather_attr<true, false, true>();
+            set_gather_attr<false, true, true>();
+            set_gather_attr<true, true, true>();
             (void)hipGetLastError();
             (void)hipSetDevice(cur);
         });
@@ -627,7 +638,9 @@ void launch_gather(int32_t device, const gather_args & a, hipStream_t st) {
     const uint32_t grid =
         static_cast<uint32_t>(a.n_splits) * static_cast<uint32_t>(a.pv.h_kv * a.head_tiles) * static_cast<uint32_t>(a.T);
     const bool kv8 = a.pv.format == kFormatKV8;
-    if (a.many) {
+    if (a.many && a.q_lo != nullptr) {
+        kv8 ? launch<true, true, true>(grid, a, st) : launch<false, true, true>(grid, a, st);
+    } else if (a.many) {
         kv8 ? launch<true, false, true>(grid, a, st) : launch<false, false, true>(grid, a, st);
     } else if (a.q_lo != nullptr) {
         kv8 ? launch<true, true, false>(grid, a, st) : launch<false, true, false>(grid, a, st);

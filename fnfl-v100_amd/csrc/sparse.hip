@@ -28,7 +28,11 @@ namespace fnkv {
 // The launch shape of `rows` rows, the deepest at position last: each row's splits, whether a wave takes several tiles,
 // and the partials of every split (a row of one split writes none, its region is unused).
 //   * Decode rows (at most kSelMaxRows): one virtual tile a wave, the row's at most 65 tiles over at most 17 splits. A
-//     step has few rows, so its time is one tile's latency, and fewer, longer splits leave the device idle.
+//     step has few rows, so its time is one tile's latency, and fewer, longer splits leave the device idle. That form
+//     holds one workgroup a CU; (row, head tile) pairs whose splits are more than the CUs (from 16 on) take the splits
+//     that one round holds, several tiles a wave: attn::attend of 5 rows of 32 heads on 8 KV heads at 3,000 cells 37.7 ->
+//     26.4 us a layer (a kernel that read whole tiles: 28.8), at 100,000 41.3 -> 29.4; without prepare and gate 33.4 ->
+//     24.6 (25.9); two rounds of workgroups a CU where they fit: 26.3.
 //   * Prompt rows: the splits that bring the launch to two workgroups a CU (what its LDS lets run at once), one from
 //     512 (row, head tile) pairs on: such rows need no partials and no merge.
 struct sparse_plan {
@@ -42,18 +46,19 @@ sparse_plan plan_sparse(const kv_pool & p, int64_t last, int32_t rows, int32_t G
     const int32_t entries = sel_shape(static_cast<int32_t>(std::min<int64_t>(last, kSelMaxCells))).K + 1;
     const int32_t full = (entries + 8 * kGatherWaves - 1) / (8 * kGatherWaves);
     pl.n_splits = full;
-    if (rows > kSelMaxRows) {
-        const int64_t pairs = int64_t(rows) * p.h_kv() * ((G + 15) / 16);
-        pl.n_splits = static_cast<int32_t>(
-            std::min<int64_t>(full, std::max<int64_t>(1, 2 * int64_t(device_cus(p.device())) / pairs)));
+    const int64_t cus = device_cus(p.device()), pairs = int64_t(rows) * p.h_kv() * ((G + 15) / 16);
+    const bool over = rows <= kSelMaxRows && pairs * full > cus;
+    if (rows > kSelMaxRows || over) {
+        pl.n_splits =
+            static_cast<int32_t>(std::min<int64_t>(full, std::max<int64_t>(1, (over ? 1 : 2) * cus / pairs)));
     }
-    pl.many = pl.n_splits < full;
+    pl.many = pl.n_splits < full || over;
     auto up16 = [](int64_t x) { return (x + 15) & ~int64_t(15); };
     const int64_t head_rows = int64_t(p.h_kv()) * G;
     pl.pml_off = rows * pl.n_splits * head_rows * kHeadDim * 4;
     // what the workspace is asked to hold: no fewer row splits than any smaller launch takes, so that one sized for a
     // caller's largest chunk serves its smaller ones (which take more splits a row)
-    const int64_t fill = std::max<int64_t>(2 * int64_t(device_cus(p.device())) / (int64_t(p.h_kv()) * ((G + 15) / 16)),
+    const int64_t fill = std::max<int64_t>(2 * cus / (int64_t(p.h_kv()) * ((G + 15) / 16)),
                                            int64_t(kSelMaxRows) * full);
     const int64_t units = std::max<int64_t>(rows, std::min<int64_t>(int64_t(rows) * full, fill));
     pl.bytes = up16(units * head_rows * (kHeadDim + 2) * 4);
@@ -136,12 +141,12 @@ int sparse_launch(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_t T
         return FNKV_ERR_ARG;
     }
     // several rows: their new cells first (a row may read an earlier row's new cell; the rows run side by side); one
-    // row: the launch writes it, by the split that reads its tile
+    // row of one tile a wave: the launch writes it, by the split that reads its tile
     if (fp != nullptr && (G > 16 || fp->rows != T)) {
         set_error(name + ": a launch that prepares its rows takes at most 16 query heads a KV head");
         return FNKV_ERR_ARG;
     }
-    if (k_new != nullptr && T > 1 && fp == nullptr) {
+    if (k_new != nullptr && (T > 1 || pl.many) && fp == nullptr) {
         if (append_enqueue(*p, slot, layer, depth, dd != nullptr ? dd->depth : nullptr, ctx, T, k_new, v_new,
                            new_dtype, st) != FNKV_OK) {
             set_error(name + ": launch failed");
@@ -164,7 +169,7 @@ int sparse_launch(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_t T
     a.q_lo = q_lo;
     if (fp != nullptr) {
         a.fp = *fp;
-    } else if (T == 1) {
+    } else if (T == 1 && !pl.many) {
         a.k_new = k_new;
         a.v_new = v_new;
         a.new_f32 = new_dtype == FNKV_F32 ? 1 : 0;

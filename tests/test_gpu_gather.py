@@ -9,6 +9,7 @@ import pytest
 import cases
 import fnkv
 import oracle as O
+import test_gpu_qsa_attend as qsa
 import test_gpu_qsp as qsp
 import test_gpu_sparse as sparse
 
@@ -65,6 +66,25 @@ def test_blocks_that_share_a_pool_tile(blocks_of_tile):
     pool, got, ref, _ = sparse.sparse_case(depth, T, seed=71,
                                            body=(words, np.array([0, 4 * words.size], np.int32), cells))
     assert cases.out_err(got, ref) <= TOL
+
+
+# decode rows whose one-tile-a-wave splits are more than the CUs: several tiles a wave (16 pairs of (row, head tile) at 17
+# splits: 272; 15: 255, the last with one tile a wave), the new cells written by the launch that prepares its rows, by a
+# prepare before it (more than 16 heads a KV head), or appended before it (one row too)
+@pytest.mark.parametrize("depth,T,hq,hkv,fmt", [
+    (3000, 3, 32, 8, fnkv.FMT_Q8_0), (2045, 5, 32, 8, fnkv.FMT_KV8), (3000, 1, 128, 16, fnkv.FMT_Q8_0),
+    (9000, 5, 96, 2, fnkv.FMT_Q8_0), (3000, 5, 12, 3, fnkv.FMT_Q8_0), (600, 5, 64, 16, fnkv.FMT_KV8)])
+def test_rows_of_many_kv_heads(depth, T, hq, hkv, fmt):
+    pool, got, ref, _ = sparse.sparse_case(depth, T, seed=depth + T + hkv, hq=hq, hkv=hkv, fmt=fmt)
+    assert np.isfinite(got).all()
+    assert cases.out_err(got, ref) <= TOL
+
+
+@pytest.mark.parametrize("depth,T,hq,hkv,fmt", [
+    (3000, 3, 32, 8, fnkv.FMT_Q8_0), (2044, 5, 32, 8, fnkv.FMT_KV8), (20001, 5, 32, 8, fnkv.FMT_Q8_0),
+    (3000, 1, 64, 16, fnkv.FMT_KV8), (2045, 5, 64, 2, fnkv.FMT_Q8_0), (3000, 5, 12, 3, fnkv.FMT_Q8_0)])
+def test_prepared_rows_of_many_kv_heads(depth, T, hq, hkv, fmt):
+    qsa.run_case(depth, T, hq, hkv, seed=depth + T + hkv, fmt=fmt, planes=True)
 
 
 # pairs (row, 16-head tile of a KV head) a launch: 17 splits a row up to 30, one split from 257 on (256 CUs, two
