@@ -30,14 +30,11 @@
 
 namespace fnkv {
 
-// Fold the splits of each (sequence, KV head, row): one workgroup a (row, 32 values); 256 threads = 8 float4
-// columns x 32 split groups. Group g folds splits g, g + 32, ... in order with a running max (all its loads
-// independent, so they are in flight together: one memory round trip), then the 32 groups fold in order in LDS
-// (deterministic: the same order for every launch).
 // The splits of sequence s that hold partials: its first s0 and count n; false when the launch refused the sequence
-// (its outputs are left as they were)
+// (its outputs are left as they were). SPARSE: the rows of a sparse launch (merge_args::sel_splits).
+template <bool SPARSE>
 __device__ __forceinline__ bool merge_splits(const merge_args & a, int32_t s, int32_t & s0, int32_t & n) {
-    if (a.sel_splits > 0) { // a sparse launch: row s's splits that held some of its virtual tiles
+    if constexpr (SPARSE) { // row s's splits that held some of its virtual tiles
         int64_t d = a.depth;
         if (a.depth_dev != nullptr) {
             d = *a.depth_dev;
@@ -63,6 +60,10 @@ __device__ __forceinline__ bool merge_splits(const merge_args & a, int32_t s, in
     return true;
 }
 
+// Fold the splits of each (sequence, KV head, row) of a dense launch with more than kRowMergeSplits splits a sequence:
+// one workgroup a (row, 32 values); 256 threads = 8 float4 columns x 32 split groups. Group g folds splits g, g + 32, ...
+// in order with a running max (all its loads independent, so they are in flight together: one memory round trip), then
+// the 32 groups fold in order in LDS (deterministic: the same order for every launch).
 __global__ __launch_bounds__(256) void merge_kernel(merge_args a) {
     __shared__ float sM[4];
     __shared__ float sL[4];
@@ -76,7 +77,7 @@ __global__ __launch_bounds__(256) void merge_kernel(merge_args a) {
     const int32_t kvh = rest % a.h_kv;
     const int32_t s = rest / a.h_kv;
     int32_t s0 = 0, n = 0;
-    if (!merge_splits(a, s, s0, n)) {
+    if (!merge_splits<false>(a, s, s0, n)) {
         return;
     }
     float m = kNegInf, l = 0.0f;
@@ -135,8 +136,7 @@ __global__ __launch_bounds__(256) void merge_kernel(merge_args a) {
         }
         const int32_t t = r / a.G, h = kvh * a.G + r % a.G;
         const int64_t row = (int64_t(s) * a.T + t) * a.hq + h;
-        const int32_t c0 = chunk * 32 + tid * 4;
-        finish4(a.fin, row, c0, As, Ls, a.fin.gate != nullptr ? finish_gate(a.fin, row, c0) : float4{});
+        finish_plain(a.fin, row, chunk * 32 + tid * 4, As, Ls);
     }
 }
 
@@ -230,11 +230,14 @@ dec_plan plan_decode(const kv_pool & p, int32_t n_seq, const int64_t * ctx, int3
     return pl;
 }
 
-// The plain fp16 output's fold: one workgroup a whole row (256 values), GRP waves = 64 float4 columns x GRP split
-// groups (one a wave: group g folds splits g, g + GRP, ... with a running max, its loads in flight together), then
-// the waves in order in LDS. An eighth of merge_kernel's workgroups: at these sizes a launch's cost is mostly the
-// dispatch of its workgroups.
-template <int GRP> __global__ __launch_bounds__(64 * GRP) void merge_row_kernel(merge_args a) {
+// The fold of at most kRowMergeSplits splits a row (every sparse launch's, most dense ones'): one workgroup a whole row
+// (256 values), GRP waves = 64 float4 columns x GRP split groups (one a wave: group g folds splits g, g + GRP, ... with a
+// running max, its loads in flight together), then the waves in order in LDS. An eighth of merge_kernel's workgroups: at
+// these sizes a launch's cost is mostly the dispatch of its workgroups. The dense, the plain sparse and the gated form
+// are instances of their own, so that a workgroup starts with only what its form needs: 8,192 rows of one split
+// (16 sequences of 500-755 cells, T = 4, 128 heads on 16 KV heads) 23.4 us as one kernel for all forms, 19.6 as its own.
+constexpr int32_t kRowMergeSplits = 96;
+template <int GRP, bool SPARSE, bool GATED> __global__ __launch_bounds__(64 * GRP) void merge_row_kernel(merge_args a) {
     __shared__ float sM[GRP];
     __shared__ float sL[GRP];
     __shared__ floatx4 sA[GRP][64];
@@ -246,12 +249,12 @@ template <int GRP> __global__ __launch_bounds__(64 * GRP) void merge_row_kernel(
     const int32_t kvh = rest % a.h_kv;
     const int32_t s = rest / a.h_kv;
     int32_t s0 = 0, n = 0;
-    if (!merge_splits(a, s, s0, n)) {
+    if (!merge_splits<SPARSE>(a, s, s0, n)) {
         return;
     }
     const int64_t row = (int64_t(s) * a.T + r / a.G) * a.hq + kvh * a.G + r % a.G;
     float4 gate = {};
-    if (a.fin.gate != nullptr && g == 0) { // requested beside the partials
+    if (GATED && g == 0) { // requested beside the partials
         gate = finish_gate(a.fin, row, c4 * 4);
     }
     float m = kNegInf, l = 0.0f;
@@ -293,22 +296,34 @@ template <int GRP> __global__ __launch_bounds__(64 * GRP) void merge_row_kernel(
         Ls = __builtin_fmaf(Ls, f0, sL[w] * f1);
         Ms = mn;
     }
-    finish4(a.fin, row, c4 * 4, As, Ls, gate);
+    if constexpr (GATED) {
+        finish_gated(a.fin, row, c4 * 4, As, Ls, gate);
+    } else {
+        finish_plain(a.fin, row, c4 * 4, As, Ls);
+    }
 }
 
 void launch_merge(const merge_args & m, hipStream_t st) {
-    // the plain fp16 output with at most 96 splits a sequence (cfg1's 67; cfg2's 128 fold faster over more threads):
-    // a workgroup a row; otherwise a workgroup a (row, 32 values)
-    int32_t most = m.sel_splits;
-    for (int32_t i = 0; m.sel_splits == 0 && i < m.n_seq; ++i) {
-        most = std::max(most, m.split0[i + 1] - m.split0[i]);
-    }
-    if (most <= 96) {
-        hipLaunchKernelGGL(merge_row_kernel<8>, dim3(static_cast<uint32_t>(m.n_seq * m.h_kv * m.R)), dim3(512), 0, st,
-                           m);
+    const dim3 rows(static_cast<uint32_t>(m.n_seq * m.h_kv * m.R));
+    if (m.sel_splits > 0) { // a sparse launch (at most 17 splits a row)
+        if (m.fin.gate != nullptr) {
+            hipLaunchKernelGGL((merge_row_kernel<8, true, true>), rows, dim3(512), 0, st, m);
+        } else {
+            hipLaunchKernelGGL((merge_row_kernel<8, true, false>), rows, dim3(512), 0, st, m);
+        }
         return;
     }
-    hipLaunchKernelGGL(merge_kernel, dim3(static_cast<uint32_t>(m.n_seq * m.h_kv * m.R * 8)), dim3(256), 0, st, m);
+    // a workgroup a row up to 96 splits a sequence (67 splits fold faster so, 128 over more threads); otherwise a
+    // workgroup a (row, 32 values)
+    int32_t most = 0;
+    for (int32_t i = 0; i < m.n_seq; ++i) {
+        most = std::max(most, m.split0[i + 1] - m.split0[i]);
+    }
+    if (most <= kRowMergeSplits) {
+        hipLaunchKernelGGL((merge_row_kernel<8, false, false>), rows, dim3(512), 0, st, m);
+    } else {
+        hipLaunchKernelGGL(merge_kernel, dim3(8 * rows.x), dim3(256), 0, st, m);
+    }
 }
 
 } // namespace fnkv

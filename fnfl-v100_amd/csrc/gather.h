@@ -111,23 +111,23 @@ __device__ __forceinline__ void gather_softmax(const floatx4 (&sc)[2], int32_t n
 }
 
 // Four values c0 .. c0 + 3 of an output row (row = token * hq + head) from their folded accumulators A and the row's
-// L; the 8 lanes of a 32-value run are consecutive and all take part. Plain: A / L as fp16. Gated (gate set,
-// fn/kernels/qsa/attend.cu:619-655's finish): A / L / (1 + exp(-gate)) in F32, with the prompt path's fp16 output or
-// the int8 activation format of the run. g4: the four gates (finish_gate), for callers that request them early.
+// L: A / L as fp16.
+__device__ __forceinline__ void finish_plain(const out_args & o, int64_t row, int32_t c0, floatx4 A, float L) {
+    const float inv = 1.0f / L;
+    uint2 pk;
+    pk.x = uint32_t(__half_as_ushort(__float2half_rn(A[0] * inv))) |
+           (uint32_t(__half_as_ushort(__float2half_rn(A[1] * inv))) << 16);
+    pk.y = uint32_t(__half_as_ushort(__float2half_rn(A[2] * inv))) |
+           (uint32_t(__half_as_ushort(__float2half_rn(A[3] * inv))) << 16);
+    *reinterpret_cast<uint2 *>(o.out + row * kHeadDim + c0) = pk;
+}
+// The gated form (fn/kernels/qsa/attend.cu:619-655's finish): A / L / (1 + exp(-gate)) in F32, with the prompt path's
+// fp16 output or the int8 activation format of the 32-value run, whose 8 lanes are consecutive and all take part. g4: the
+// four gates (finish_gate), for callers that request them early.
 __device__ __forceinline__ float4 finish_gate(const out_args & o, int64_t row, int32_t c0) {
     return *reinterpret_cast<const float4 *>(o.gate + row * o.gate_stride + c0);
 }
-__device__ __forceinline__ void finish4(const out_args & o, int64_t row, int32_t c0, floatx4 A, float L, float4 g4) {
-    if (o.gate == nullptr) {
-        const float inv = 1.0f / L;
-        uint2 pk;
-        pk.x = uint32_t(__half_as_ushort(__float2half_rn(A[0] * inv))) |
-               (uint32_t(__half_as_ushort(__float2half_rn(A[1] * inv))) << 16);
-        pk.y = uint32_t(__half_as_ushort(__float2half_rn(A[2] * inv))) |
-               (uint32_t(__half_as_ushort(__float2half_rn(A[3] * inv))) << 16);
-        *reinterpret_cast<uint2 *>(o.out + row * kHeadDim + c0) = pk;
-        return;
-    }
+__device__ __forceinline__ void finish_gated(const out_args & o, int64_t row, int32_t c0, floatx4 A, float L, float4 g4) {
     const float gr[4] = {g4.x, g4.y, g4.z, g4.w};
     float y[4];
 #pragma unroll
@@ -160,6 +160,14 @@ __device__ __forceinline__ void finish4(const out_args & o, int64_t row, int32_t
         (uint32_t(uint8_t(q[3])) << 24);
     if ((c0 & 31) == 0) {
         *reinterpret_cast<float2 *>(o.act_scales + (row * 8 + c0 / 32) * 2) = float2{ds[0], ds[1]};
+    }
+}
+// either, by the launch's outputs
+__device__ __forceinline__ void finish4(const out_args & o, int64_t row, int32_t c0, floatx4 A, float L, float4 g4) {
+    if (o.gate == nullptr) {
+        finish_plain(o, row, c0, A, L);
+    } else {
+        finish_gated(o, row, c0, A, L, g4);
     }
 }
 
