@@ -34,7 +34,10 @@ def launch(ctxs, T, hq, hkv, seed, dev_slack=0, shrink=0, fmt=fnkv.FMT_Q8_0):
     q16 = cases.queries(seed, (len(ctxs), T, hq, 256))
     q = torch.from_numpy(q16).cuda()
     out = torch.full_like(q, float("nan"))
-    ws = torch.zeros(pool.decode_ws_bytes(bound, T, hq) - shrink, dtype=torch.uint8, device="cuda")
+    held = pool.decode_ws_bytes(bound, T, hq) - shrink
+    buf = torch.zeros(held + shrink + (1 << 20), dtype=torch.uint8, device="cuda")
+    buf[held:] = 0x5a  # the bytes behind the workspace stay as they are
+    ws = buf[:held]
     slots = list(range(len(ctxs)))
     if dev_slack:
         err = torch.zeros(1, dtype=torch.int32, device="cuda")
@@ -44,6 +47,7 @@ def launch(ctxs, T, hq, hkv, seed, dev_slack=0, shrink=0, fmt=fnkv.FMT_Q8_0):
     else:
         pool.decode(slots, ctxs, T, 0, q, out, ws)
         torch.cuda.synchronize()
+    assert int((buf[held:] != 0x5a).sum()) == 0
     return q16, out.cpu().numpy(), rows
 
 
@@ -70,7 +74,7 @@ def test_fine_splits(ctxs, dev_slack, T):
 @pytest.mark.parametrize("T", [1, 5])
 def test_a_workspace_below_the_fine_plans(T):
     ctxs = [4099]
-    for shrink in (1, 8192):
+    for shrink in (257, 8192):  # (the size asked for holds 256 bytes more than the plan: 257 leaves one byte less)
         q16, got, rows = launch(ctxs, T, 16, 2, 920 + T, shrink=shrink)
         check(q16, got, rows, ctxs, 16, 2, [0, 1])
     with pytest.raises(fnkv.FnkvError):  # below the coarser plan's 17 splits as well
@@ -98,7 +102,10 @@ def test_a_workspace_for_deeper_contexts_serves_shorter_ones(deep, T_deep):
         g = torch.Generator(device="cuda").manual_seed(970 + s)
         k, v = (torch.randn((c, hkv, 256), generator=g, device="cuda").half() for _ in range(2))
         pool.append(s, 0, 0, k, v)
-    ws = torch.zeros(pool.decode_ws_bytes(deep, T_deep, hq), dtype=torch.uint8, device="cuda")
+    held = pool.decode_ws_bytes(deep, T_deep, hq)
+    buf = torch.zeros(held + (8 << 20), dtype=torch.uint8, device="cuda")
+    buf[held:] = 0x5a  # the bytes behind the workspace stay as they are
+    ws = buf[:held]
     calls = [[c] for c in range(T_deep, deep[0], 6007)]
     calls += [[c] for c in (22017, 32768, 33000, 65505, 98305, 131041, 131072, 196577) if c < deep[0]]
     calls += [[max(T_deep, int(c * x)) for c in deep] for x in (0.999, 0.95, 0.7, 0.51, 0.3, 0.1)]
@@ -112,8 +119,9 @@ def test_a_workspace_for_deeper_contexts_serves_shorter_ones(deep, T_deep):
             pool.decode(slots, ctxs, T, 0, q, got, ws)
             pool.decode(slots, ctxs, T, 0, q, own, torch.zeros(n, dtype=torch.uint8, device="cuda"))
             torch.cuda.synchronize()
-            smaller += n > ws.numel()
+            smaller += n > held
             assert float((got.float() - own.float()).abs().max()) <= 2 * TOL, (ctxs, T)
+    assert int((buf[held:] != 0x5a).sum()) == 0
     print(f"{smaller} of {2 * len(calls)} calls ask for more than the workspace")
     assert smaller > 0
 
