@@ -20,7 +20,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <cstdlib>
 #include <string>
 
 namespace fnkv {
@@ -33,8 +32,8 @@ namespace fnkv {
 //     that one round holds, several tiles a wave: attn::attend of 5 rows of 32 heads on 8 KV heads at 3,000 cells 37.7 ->
 //     26.4 us a layer (a kernel that read whole tiles: 28.8), at 100,000 41.3 -> 29.4; without prepare and gate 33.4 ->
 //     24.6 (25.9); two rounds of workgroups a CU where they fit: 26.3.
-//   * Prompt rows: the splits that bring the launch to two workgroups a CU (what its LDS lets run at once), one from
-//     512 (row, head tile) pairs on: such rows need no partials and no merge.
+//   * Prompt rows: the splits that bring the launch to at most two workgroups a CU (what its LDS lets run at once): one
+//     where the (row, head tile) pairs are more than the CUs. Such rows need no partials and no merge.
 struct sparse_plan {
     int32_t n_splits = 0;
     bool many = false;
@@ -56,11 +55,11 @@ sparse_plan plan_sparse(const kv_pool & p, int64_t last, int32_t rows, int32_t G
     auto up16 = [](int64_t x) { return (x + 15) & ~int64_t(15); };
     const int64_t head_rows = int64_t(p.h_kv()) * G;
     pl.pml_off = rows * pl.n_splits * head_rows * kHeadDim * 4;
-    // what the workspace is asked to hold: no fewer row splits than any smaller launch takes, so that one sized for a
-    // caller's largest chunk serves its smaller ones (which take more splits a row)
+    // what the workspace is asked to hold: no fewer row splits than any smaller launch writes, so that one sized for a
+    // caller's largest chunk serves its smaller ones (which take more splits a row); rows of one split write none
     const int64_t fill = std::max<int64_t>(2 * cus / (int64_t(p.h_kv()) * ((G + 15) / 16)),
                                            int64_t(kSelMaxRows) * full);
-    const int64_t units = std::max<int64_t>(rows, std::min<int64_t>(int64_t(rows) * full, fill));
+    const int64_t units = std::min<int64_t>(int64_t(rows) * full, fill);
     pl.bytes = up16(units * head_rows * (kHeadDim + 2) * 4);
     return pl;
 }

@@ -107,3 +107,22 @@ def test_prompt_workspace_serves_smaller_chunks(hq, hkv):
         for pos0 in (0, 100, 2000, 40000):
             assert 0 < pool.qsp_ws_bytes(pos0, a, hq) <= pool.qsp_ws_bytes(pos0, b, hq)
             assert pool.qsp_ws_bytes(pos0, a, hq) <= pool.qsp_ws_bytes(pos0 + 1000, a, hq)
+    # and no more than the partials that some launch writes: rows of several splits fill two workgroups a CU at most (256
+    # CUs), five rows take 17 splits each, and rows of one split write none
+    head_tiles = hkv * -(-hq // hkv // 16)
+    assert pool.qsp_ws_bytes(40000, 4096, hq) <= max(512 // head_tiles, 5 * 17) * hq * 258 * 4 + 16
+
+
+@pytest.mark.parametrize("rows,hq,h_kv", [(6, 12, 1), (30, 12, 1), (100, 40, 2), (256, 12, 1), (257, 12, 1)])
+def test_prompt_rows_stay_within_their_workspace(rows, hq, h_kv, monkeypatch):
+    attend = fnkv.Pool.qsp_attend
+
+    def guarded(pool, slot, layer, pos0, qfull, *more, **kw):
+        need = pool.qsp_ws_bytes(pos0, rows, hq)
+        buf = torch.full((need + (8 << 20),), 0x5a, dtype=torch.uint8, device="cuda")
+        attend(pool, slot, layer, pos0, qfull, *more, ws=buf[:need], **kw)
+        assert int((buf[need:] != 0x5a).sum()) == 0
+
+    monkeypatch.setattr(fnkv.Pool, "qsp_attend", guarded)
+    _, o32, err, ref = qsp.run_attend(3000, rows, hq, h_kv, seed=rows + hq)
+    assert err == 0 and float(np.abs(o32.astype(np.float64) - ref).max()) <= TOL
