@@ -28,7 +28,7 @@ struct dec_args {
     float * pml;        // [total_splits][h_kv][R][2] partial (m, l), base-2 domain
     float c2;           // scale * log2(e)
     int32_t layer, T, G, hq, R, n_seq, split_tokens;
-    // dense: 1 when a sequence's n splits stride over its tiles (split j takes tiles j, j + n, ...; at most 64 a
+    // dense: 1 when a sequence's n splits stride over its tiles (split j takes tiles j, j + n, ...; at most 128 a
     // split), 0 when split j takes the cells j split_tokens .. + split_tokens - 1
     int32_t strided;
     int32_t slot[FNKV_MAX_SEQS];
@@ -264,8 +264,8 @@ constexpr int32_t kFineSplit = 128;
 constexpr int64_t kAnySplits = int64_t(1) << 40;
 struct split_choice {
     int32_t cells = 0; // a split's
-    // the best split of at most 64 tiles: the workspace asked for holds its partials too, so a launch that takes longer
-    // splits is refused by the same workspaces
+    // the best split of at most 64 tiles: the workspace asked for holds its partials too, so the size asked for is no
+    // smaller where a launch takes longer splits (fewer partials)
     int32_t asked = 0;
 };
 split_choice choose_split_stream(int32_t n_seq, const int64_t * ctx, int32_t h_kv, int32_t cus, int32_t NT, bool fine,
@@ -279,7 +279,7 @@ struct dev_depth {
 };
 // host: a sparse launch of decode rows over the pool (sparse.hip), with gated outputs when `gate` is set.
 // dd set: `depth` is not read; the plan (grid, workspace) follows from dd->max_cells. q_lo set: q's fp16 low parts
-// beside q (dec_args::q_lo), 16-byte aligned
+// beside q (gather_args::q_lo), 16-byte aligned
 int sparse_launch(const fnkv_pool * pool, int32_t slot, int64_t depth, int32_t T, int32_t layer, int32_t hq, float scale,
                   const void * q, const void * body, const void * offsets, const void * k_new, const void * v_new,
                   int32_t new_dtype, void * out, const out_args * gate, void * ws, int64_t ws_bytes,

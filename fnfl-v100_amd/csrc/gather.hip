@@ -16,16 +16,19 @@
 //     v_mfma_f32_16x16x32_f16 reads (K: 8 loads of 16 B; V: 16 of 12 B, of which 8 are its cells'), and the scores, the
 //     softmax and PV run on the virtual tile as on a stored one. Entry e of the body is cell group e of virtual tile
 //     e / 8, so no workgroup builds a list: a lane's block is one body word and one page-table word.
-//   * A workgroup of 4 waves (one a SIMD; two workgroups a CU for prompt rows) owns (row, up to 16 query heads of a KV head, split):
-//     wave w of split s takes virtual tiles 4 s + w, + 4 n_splits, ... Decode rows launch enough splits for one tile a
-//     wave (at most 17 splits of a row's 65 tiles) where those are at most one workgroup a CU; prompt rows split only while the rows alone do not fill the device,
-//     and a row of one split is finished here, without partials or a merge.
+//   * A workgroup of 4 waves (one a SIMD; two workgroups a CU for prompt rows) owns (row, up to 16 query heads of a KV
+//     head, split): wave w of split s takes virtual tiles 4 s + w, + 4 n_splits, ... Decode rows launch enough splits for
+//     one tile a wave (at most 17 splits of a row's 65 tiles) where those are at most one workgroup a CU; prompt rows split
+//     only while the rows alone do not fill the device, and a row of one split is finished here, without partials or a
+//     merge.
 //   * A tile's K and scales are requested while the previous tile is in its softmax and PV, its V while the next
 //     scores run; every block of the wave's tiles is resolved (body word, then page) before the first.
 //   * The workgroups are laid out so that an XCD's share of them is consecutive rows: a prompt's neighbouring rows
 //     select much the same blocks and find them in that XCD's L2.
 // What bounds it: decode rows, latency (depth word, body, page table, blocks, then the fold and the merge launch);
-// prompt rows, VALU issue (565 instructions and 52 MFMAs a virtual tile, ~85% of the loop's cycles).
+// prompt rows, VALU issue (the loop: about 455 instructions and 52 MFMAs a virtual tile, 84 more where it moves the
+// softmax reference; with the rest of the kernel 619 and 52.5, issued in 76% of the cycles that a SIMD holds two waves; the
+// blocks come from L2 at about 10 TB/s).
 // Measured against a kernel that rebuilt each row's tile list in LDS and read whole tiles (kernel trace, us; 12 heads
 // on one KV head unless said): 1,000 prompt rows at 40,000 cells 128.6 + no merge (1,398 in two chunks + 198 of
 // merges); attn::attend rows at 196,608 cells, 3 rows 12.4 + 4.9 merge (20.5 + 6.1); 16 heads on 2 KV heads, one KV8

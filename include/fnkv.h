@@ -356,13 +356,14 @@ int fnkv_qsp_attend(const fnkv_qsp_attend_args * a, void * stream);
 
 /* ---- chunked-prefill attention (fn/kernels/qsa/qsa_prompt.h:106-124 qsp_attend) ---- */
 
-/* the workspace a prefill launch of this shape uses (bytes; 0: none; -1: a shape outside the contract) */
+/* the workspace a prefill launch of this shape uses (bytes; 0: none; -1: a shape outside the contract). A smaller chunk
+ * can use more than a larger one: for chunks of several sizes take the largest */
 int64_t fnkv_prefill_workspace_bytes(const fnkv_pool * pool, int64_t ctx, int32_t rows, int32_t hq);
 
 /* Causal attention of `rows` query tokens (positions ctx - rows .. ctx - 1 of the slot, already appended) over the
- * slot's cells 0 .. ctx - 1 of `layer`, on the matrix cores with fp32 accumulation: K and V (code x scale) as exact
- * hi + lo fp16 operands, P as hi + lo fp16 (the reference's prompt attention rounds its operands to fp16 once,
- * qsa_prompt.h:55-58; this keeps ~22 bits a product). q: fp16 [rows][hq][256], out: fp16 [rows][hq][256].
+ * slot's cells 0 .. ctx - 1 of `layer`, on the matrix cores with fp32 accumulation: the K and V codes exactly, K's
+ * scales on the fp32 scores, P times V's scales as hi + lo fp16 (the reference's prompt attention rounds its operands to
+ * fp16 once, qsa_prompt.h:55-58; this keeps ~19 bits a product or more). q: fp16 [rows][hq][256], out: fp16 [rows][hq][256].
  * ws: fnkv_prefill_workspace_bytes bytes of device memory (no zeroing needed) for the key-split partials when the
  * query rows alone do not fill the device; smaller: the splits that it holds; null: one split, no workspace. The GQA
  * group hq / h_kv must divide 256 (a workgroup's query rows). */
